@@ -1,0 +1,308 @@
+// Linear-layer GEMM for 65 and more tokens: y = x W^T with the layer's own
+// epilogue (bias, residual, or SiLU(gate) * up), 16-bit operands, fp32 sums.
+//
+// What bounds it: from about a thousand tokens the matrix cores (under their
+// load the chip is power limited), below that the weight stream and the number
+// of CUs that have a tile.  A workgroup of RW x CW waves owns a BM x BN tile
+// and runs the ring of bfa_gemm.h.  The tile sizes differ in how well they fill
+// the 256 CUs, which decides more than the loop does (Llama-3-8B, 300 tokens:
+// gate_up on 128 x 256 tiles is 336 tiles, two rounds of which the second is
+// nearly empty; on 160 x 256 it is one round of 224).  What whole rounds of
+// tiles do not fill is split over K: the last tiles go to several workgroups
+// each, whose fp32 partial tiles linear_reduce_kernel sums, in split order, into
+// the same epilogue.
+//
+// Measured against the projection GEMM's tiles with linear epilogues, which
+// these replace (Llama-3-8B, weights from HBM, same box): gate_up+SiLU*mul 94 ->
+// 56 us at 100 tokens, 158 -> 76 us at 300 (927 TFLOP/s; a plain library GEMM
+// 76 us), 1235 -> 1119 us at 6000; down_proj+residual 165 -> 35 us, 153 -> 52 us
+// and 728 -> 572 us (1232 TFLOP/s).
+#include "bfa_gemm.h"
+#include "bfa_host.h"
+#include "bfa_linear.h"
+#include "bfa_qkv.h"
+
+namespace bfa {
+
+// Output columns of the wave's 64 weight rows: row 16 j + 4 g + v feeds
+//   plain    column 16 g + 4 j + v                          (a lane: 16 consecutive)
+//   SwiGLU   gate (j < 2) or up column 8 g + 4 (j % 2) + v  (a lane: 8 of each)
+// so that a lane's values are neighbours in one token's output row and go out in
+// 16-byte stores straight from the accumulators.
+template <bool SWIGLU>
+__device__ __forceinline__ int64_t lin_weight_row(const LinArgs& q, int64_t n0, int c) {
+  const int w = c >> 6, j = (c >> 4) & 3, g = (c >> 2) & 3, v = c & 3;
+  if constexpr (SWIGLU) {
+    const int64_t o = min(n0 + w * 32 + g * 8 + (j & 1) * 4 + v, q.n - 1);
+    return j < 2 ? o : q.n + o;
+  } else {
+    return min(n0 + w * 64 + g * 16 + j * 4 + v, q.n - 1);
+  }
+}
+
+// Eight neighbouring outputs (columns c .. c + 7) of one token.  SAME: proj_dt,
+// out_dt and res_dt are DT, mid_dt DT or fp32, vec rows and n a multiple
+// of 8; otherwise the dtypes and bounds are the call's.
+template <int DT, bool SAME, bool SWIGLU>
+__device__ __forceinline__ void lin_out8(const LinArgs& q, int64_t row, int64_t c, const float (&a)[8],
+                                         const float (&u)[8], const uint4& res) {
+  using E = Elem<DT>;
+  if (c >= q.n) return;
+  float y[8];
+  if constexpr (SAME) {
+    const uint32_t rw[4] = {res.x, res.y, res.z, res.w};
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      if constexpr (SWIGLU) {
+        y[t] = E::round(silu_fast(E::round(a[t]))) * E::round(u[t]);
+      } else {
+        float v = a[t];
+        if (q.bias) v = v + load_any(q.bias, q.bias_dt, c + t);
+        v = E::round(v);
+        if (q.res) v = v + E::to_f32(static_cast<uint16_t>((t & 1) ? rw[t >> 1] >> 16 : rw[t >> 1] & 0xffffu));
+        y[t] = v;
+      }
+    }
+    store8<DT>(static_cast<uint16_t*>(q.out) + row * q.ldo + c, y);
+  } else {
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      if constexpr (SWIGLU) {
+        y[t] = round_to(silu_fast(round_to(a[t], q.proj_dt)), q.proj_dt) * round_to(u[t], q.proj_dt);
+      } else {
+        const int64_t cc = min(c + t, q.n - 1);
+        float v = a[t];
+        if (q.bias) v = v + load_any(q.bias, q.bias_dt, cc);
+        v = round_to(v, q.proj_dt);
+        v = v + (q.res ? load_any(q.res, q.res_dt, row * q.ldr + cc) : 0.f);
+        y[t] = round_to(v, q.mid_dt);
+      }
+    }
+    if (q.vec && c + 8 <= q.n) {
+      if (q.out_dt == BFA_DTYPE_BF16) store8<BFA_DTYPE_BF16>(static_cast<uint16_t*>(q.out) + row * q.ldo + c, y);
+      else if (q.out_dt == BFA_DTYPE_F16) store8<BFA_DTYPE_F16>(static_cast<uint16_t*>(q.out) + row * q.ldo + c, y);
+      else store8<BFA_DTYPE_F32>(static_cast<float*>(q.out) + row * q.ldo + c, y);
+    } else {
+#pragma unroll
+      for (int t = 0; t < 8; ++t)
+        if (c + t < q.n) store_any(q.out, q.out_dt, row * q.ldo + c + t, y[t]);
+    }
+  }
+}
+
+// One token's 16 projection values of a lane; c0 its first output column.
+template <int DT, bool SAME, bool SWIGLU>
+__device__ __forceinline__ void lin_finish(const LinArgs& q, int64_t row, int64_t c0, const gemm_f32x4_t (&acc)[4],
+                                           const uint4 (&res)[2]) {
+  const float lo[8] = {acc[0][0], acc[0][1], acc[0][2], acc[0][3], acc[1][0], acc[1][1], acc[1][2], acc[1][3]};
+  const float hi[8] = {acc[2][0], acc[2][1], acc[2][2], acc[2][3], acc[3][0], acc[3][1], acc[3][2], acc[3][3]};
+  if constexpr (SWIGLU) {
+    lin_out8<DT, SAME, true>(q, row, c0, lo, hi, res[0]);
+  } else {
+    lin_out8<DT, SAME, false>(q, row, c0, lo, lo, res[0]);
+    lin_out8<DT, SAME, false>(q, row, c0 + 8, hi, hi, res[1]);
+  }
+}
+
+// The lane's residual elements, ahead of their use (columns past n are clamped;
+// their results are not stored).
+template <bool SAME, bool SWIGLU>
+__device__ __forceinline__ void lin_residual(const LinArgs& q, int64_t row, int64_t c0, uint4 (&res)[2]) {
+  res[0] = res[1] = make_uint4(0, 0, 0, 0);
+  if constexpr (SAME && !SWIGLU) {
+    if (q.res) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        res[h] = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(q.res) + row * q.ldr +
+                                                 min(c0 + 8 * h, q.n - 8));
+    }
+  }
+}
+
+// The first q.full workgroups take whole tiles; each of the tiles after those
+// goes to q.splits workgroups, one K range each (q.full is a multiple of 8 or
+// covers every tile, so both parts keep their XCDs).
+template <int MA, int RW, int CW, int NS, int DT, bool SAME, bool SWIGLU>
+__global__ __launch_bounds__(RW * CW * 64, 2) void linear_gemm_kernel(LinArgs q) {
+  using T = GemmTile<MA, RW, CW, NS, DT>;
+  __shared__ uint4 lds[T::LDS_U4];
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = wid / CW, wc = wid % CW;
+  const int b = blockIdx.x;
+  const bool part = b >= q.full;
+  const int rest = q.tiles_m * q.tiles_n - q.full;
+  const int u = part ? gemm_band(b - q.full, rest * q.splits) : gemm_band(b, q.full);
+  const int split = part ? u / rest : 0, tile = part ? q.full + (u - split * rest) : u, ns = part ? q.splits : 1;
+  int tm, tn;
+  gemm_tile(q.tiles_m, q.tiles_n, tile, tm, tn);
+  const int64_t m0 = static_cast<int64_t>(tm) * T::BM;
+  const int64_t n0 = static_cast<int64_t>(tn) * (SWIGLU ? T::BN / 2 : T::BN);
+  const int k0 = static_cast<int>(static_cast<int64_t>(q.kt) * split / ns);
+  const int nk = static_cast<int>(static_cast<int64_t>(q.kt) * (split + 1) / ns) - k0;
+  typename T::Acc acc;
+  T::run(acc, lds, q.a + static_cast<int64_t>(k0) * 64, q.w + static_cast<int64_t>(k0) * 64, q.m, q.lda, q.ldw, m0, nk,
+         wid, lane, [&](int c) { return lin_weight_row<SWIGLU>(q, n0, c); }, [] {});
+
+  const int64_t wm0 = m0 + wr * MA * 16;
+  if (part) {
+    gemm_store_part<MA, 4>(q.part, static_cast<int64_t>(tile - q.full) * q.splits + split, T::NW, wid, lane,
+                           static_cast<int>(cdiv(q.m - wm0, 16)), acc);
+    return;
+  }
+  const int64_t c0 = n0 + (SWIGLU ? wc * 32 + (lane >> 4) * 8 : wc * 64 + (lane >> 4) * 16);
+  const int64_t r0 = wm0 + (lane & 15);
+  // the residual rows of half the blocks are requested together (of all of
+  // them, the 256 x 256 tile spills 16 registers)
+  constexpr int H = (MA + 1) / 2;
+#pragma unroll
+  for (int h = 0; h < MA; h += H) {
+    uint4 res[H][2];
+#pragma unroll
+    for (int i = 0; i < H; ++i) lin_residual<SAME, SWIGLU>(q, min(r0 + (h + i) * 16, q.m - 1), c0, res[i]);
+#pragma unroll
+    for (int i = 0; i < H && h + i < MA; ++i)
+      if (r0 + (h + i) * 16 < q.m) lin_finish<DT, SAME, SWIGLU>(q, r0 + (h + i) * 16, c0, acc[h + i], res[i]);
+  }
+}
+
+// One wave per 16-token x 64-column block of a split tile.
+template <int DT, bool SAME, bool SWIGLU>
+__global__ __launch_bounds__(256) void linear_reduce_kernel(LinArgs q, int ma, int rw, int cw, int items) {
+  const int item = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (item >= items) return;
+  const int lane = threadIdx.x & 63;
+  const int per = rw * cw * ma, rest = item / per, in = item - rest * per;
+  const int w = in / ma, i = in - w * ma, wr = w / cw, wc = w - wr * cw;
+  int tm, tn;
+  gemm_tile(q.tiles_m, q.tiles_n, q.full + rest, tm, tn);
+  const int64_t row0 = (static_cast<int64_t>(tm) * rw * ma + wr * ma + i) * 16, row = row0 + (lane & 15);
+  if (row0 >= q.m) return;  // no partials there
+  const int64_t c0 = SWIGLU ? (static_cast<int64_t>(tn) * cw + wc) * 32 + (lane >> 4) * 8
+                            : (static_cast<int64_t>(tn) * cw + wc) * 64 + (lane >> 4) * 16;
+  uint4 res[2];
+  lin_residual<SAME, SWIGLU>(q, min(row, q.m - 1), c0, res);
+  gemm_f32x4_t acc[4];
+  const int64_t stride = static_cast<int64_t>(per) * 256;
+  gemm_sum_part(reinterpret_cast<const gemm_f32x4_t*>(q.part) + (static_cast<int64_t>(rest) * q.splits * per + in) * 256 + lane,
+                stride, q.splits, acc);
+  if (row < q.m) lin_finish<DT, SAME, SWIGLU>(q, row, c0, acc, res);
+}
+
+// ------------------------------------------------------------------- host
+namespace {
+
+// The tiles, and a stage's time on a full chip (BM x BN x 64, 256 workgroups,
+// measured at 6000 tokens with K = 4096 and 14336): the planner compares tiles
+// by rounds x stages x this.  The wide tiles do more per LDS byte (0.95 us for
+// 128 x 256 against 1.55 for twice the work), the small ones fill a short grid.
+struct LinTile {
+  int ma, rw, cw;
+  double stage_us;
+};
+constexpr LinTile kTiles[] = {
+    {8, 2, 4, 1.55},  // 0: 256 x 256, 2 stages
+    {6, 2, 4, 1.30},  // 1: 192 x 256, 2
+    {5, 2, 4, 1.12},  // 2: 160 x 256, 3
+    {4, 2, 4, 0.95},  // 3: 128 x 256, 3
+    {4, 4, 2, 0.96},  // 4: 256 x 128, 3
+    {3, 4, 2, 0.75},  // 5: 192 x 128, 4
+    {2, 4, 2, 0.58},  // 6: 128 x 128, 5
+    {1, 4, 2, 0.38},  // 7:  64 x 128, 6
+};
+constexpr int kNumTiles = static_cast<int>(sizeof(kTiles) / sizeof(kTiles[0]));
+
+template <int MA, int RW, int CW, int NS, int DT, bool SAME>
+void launch_tile(const LinArgs& q, hipStream_t st) {
+  const int rest = q.tiles_m * q.tiles_n - q.full;
+  const dim3 grid(static_cast<unsigned>(q.full + rest * q.splits)), block(RW * CW * 64);
+  if (q.swiglu) hipLaunchKernelGGL((linear_gemm_kernel<MA, RW, CW, NS, DT, SAME, true>), grid, block, 0, st, q);
+  else hipLaunchKernelGGL((linear_gemm_kernel<MA, RW, CW, NS, DT, SAME, false>), grid, block, 0, st, q);
+}
+
+template <int DT, bool SAME>
+void launch_form(const LinPlan& p, const LinArgs& q, hipStream_t st) {
+  switch (p.tile) {
+    case 0: launch_tile<8, 2, 4, 2, DT, SAME>(q, st); break;
+    case 1: launch_tile<6, 2, 4, 2, DT, SAME>(q, st); break;
+    case 2: launch_tile<5, 2, 4, 3, DT, SAME>(q, st); break;
+    case 3: launch_tile<4, 2, 4, 3, DT, SAME>(q, st); break;
+    case 4: launch_tile<4, 4, 2, 3, DT, SAME>(q, st); break;
+    case 5: launch_tile<3, 4, 2, 4, DT, SAME>(q, st); break;
+    case 6: launch_tile<2, 4, 2, 5, DT, SAME>(q, st); break;
+    default: launch_tile<1, 4, 2, 6, DT, SAME>(q, st); break;
+  }
+  const int rest = q.tiles_m * q.tiles_n - q.full;
+  if (rest > 0) {
+    const LinTile& t = kTiles[p.tile];
+    const int items = rest * t.rw * t.cw * t.ma;
+    const dim3 grid(static_cast<unsigned>(cdiv(items, 4)));
+    if (q.swiglu) hipLaunchKernelGGL((linear_reduce_kernel<DT, SAME, true>), grid, dim3(256), 0, st, q, t.ma, t.rw, t.cw, items);
+    else hipLaunchKernelGGL((linear_reduce_kernel<DT, SAME, false>), grid, dim3(256), 0, st, q, t.ma, t.rw, t.cw, items);
+  }
+}
+
+}  // namespace
+
+// Each tile is weighed with every tile whole and, where the last round is not
+// full, with that round's tiles split over K as often as the CUs allow: rounds
+// times (stages x stage_us + 4 us of fill and epilogue), and for split tiles the
+// second launch and the partials' round trip.  Overrides: BFA_TUNE_LINEAR_TILE,
+// BFA_TUNE_LINEAR_SPLITS.
+LinPlan linear_plan(int64_t m, int64_t n, int64_t k, bool swiglu, bool split) {
+  const int ot = tuning(BFA_TUNE_LINEAR_TILE), os = tuning(BFA_TUNE_LINEAR_SPLITS);
+  const int64_t kt = k / 64;
+  LinPlan best{};
+  double cost = 0;
+  for (int id = 0; id < kNumTiles; ++id) {
+    if (ot >= 0 && ot < kNumTiles && id != ot) continue;
+    const LinTile& t = kTiles[id];
+    LinPlan p{};
+    p.tile = id;
+    p.tiles_m = cdiv(m, 16 * t.ma * t.rw);
+    p.tiles_n = cdiv(n, (swiglu ? 32 : 64) * t.cw);
+    const int64_t tiles = p.tiles_m * p.tiles_n, rounds = tiles / 256, rest = tiles % 256;
+    p.full = static_cast<int>(tiles);
+    p.splits = 1;
+    double c = static_cast<double>(rounds + (rest > 0)) * (kt * t.stage_us + 4.0);
+    int64_t s = rest > 0 ? 256 / rest : 1;
+    if (os >= 1) s = os;
+    s = std::min<int64_t>(std::min<int64_t>(s, kt), 32);
+    if (split && rest > 0 && s > 1) {
+      const int64_t bytes = rest * s * t.rw * t.cw * t.ma * 4 * 64 * 16;
+      const double cs = static_cast<double>(rounds) * (kt * t.stage_us + 4.0) + cdiv(rest * s, 256) * (cdiv(kt, s) * t.stage_us + 4.0) +
+                        4.0 + static_cast<double>(bytes) / 3.0e6;
+      if (cs < c || os > 1) {
+        c = cs;
+        p.full = static_cast<int>(rounds * 256);
+        p.splits = static_cast<int>(s);
+        p.part_bytes = bytes;
+      }
+    }
+    if (best.splits == 0 || c < cost) {
+      best = p;
+      cost = c;
+    }
+  }
+  return best;
+}
+
+void launch_linear_gemm(const LinPlan& p, LinArgs q, int dt, hipStream_t st) {
+  q.tiles_m = static_cast<int>(p.tiles_m);
+  q.tiles_n = static_cast<int>(p.tiles_n);
+  q.full = p.full;
+  q.splits = p.splits;
+  q.kt = static_cast<int>(q.k / 64);
+  // (the sum's own rounding is fp32's, none, or the output's)
+  const bool same = q.vec && q.n % 8 == 0 && q.proj_dt == dt && q.out_dt == dt &&
+                    (q.swiglu || ((q.mid_dt == dt || q.mid_dt == BFA_DTYPE_F32) && (!q.res || q.res_dt == dt)));
+  if (dt == BFA_DTYPE_BF16) {
+    if (same) launch_form<BFA_DTYPE_BF16, true>(p, q, st);
+    else launch_form<BFA_DTYPE_BF16, false>(p, q, st);
+  } else {
+    if (same) launch_form<BFA_DTYPE_F16, true>(p, q, st);
+    else launch_form<BFA_DTYPE_F16, false>(p, q, st);
+  }
+}
+
+}  // namespace bfa

@@ -45,6 +45,7 @@
 #include "bfa_device.h"
 #include "bfa_host.h"
 #include "bfa_internal.h"
+#include "bfa_linear.h"
 #include "bfa_qkv.h"
 
 namespace bfa {
@@ -2621,12 +2622,6 @@ static int fused_edt(const QkvEpi& e) {
   return EDT_RT;
 }
 
-static int linear_edt(const QkvEpi& e) {
-  if (edt_forced_rt()) return EDT_RT;
-  return (e.qkv_dt == BFA_DTYPE_BF16 && e.mid_dt == BFA_DTYPE_BF16 && e.out_dt == BFA_DTYPE_BF16)
-             ? EDT_BF16 : EDT_RT;
-}
-
 template <int BM, int BN, int WM, int NS, int BK, bool BF16, bool DIRECT, int HD>
 static void launch_fused_edt(unsigned grid, dim3 block, int edt, const GemmArgs& g, const QkvEpi& e,
                              hipStream_t st) {
@@ -2700,48 +2695,17 @@ static void launch_prefill_narrow_hd(const GemmArgs& g, const QkvEpi& e, hipStre
   hipLaunchKernelGGL((qkv_gemm_kernel<128, 64, 32, 64, BF16, EPI_FUSED, HD, true, 4, 32>), grid, block, 0, st, g, e);
 }
 
-// The linear fusions: same tiles, EPI_LINEAR or EPI_SWIGLU epilogue.
-template <int BM, int BN, int WM, int NS, int BK, bool BF16, bool DIRECT>
-static void launch_linear_tile(const GemmArgs& g, const QkvEpi& e, bool swiglu, hipStream_t st) {
-  const int64_t bno = swiglu ? BN / 2 : BN;
-  const unsigned grid = persistent_grid(cdiv(g.m, BM) * cdiv(g.n, bno), BM == 256 && BN == 256);
-  const dim3 block((BM / WM) * (BN / 128) * 64);
-  if constexpr (BF16 && DIRECT) {
-    if (linear_edt(e) == EDT_BF16) {
-      if (swiglu)
-        hipLaunchKernelGGL((qkv_gemm_kernel<BM, BN, WM, 128, BF16, EPI_SWIGLU, 128, DIRECT, NS, BK, EDT_BF16>),
-                           dim3(grid), block, 0, st, g, e);
-      else
-        hipLaunchKernelGGL((qkv_gemm_kernel<BM, BN, WM, 128, BF16, EPI_LINEAR, 128, DIRECT, NS, BK, EDT_BF16>),
-                           dim3(grid), block, 0, st, g, e);
-      return;
-    }
-  }
-  if (swiglu) {
-    hipLaunchKernelGGL((qkv_gemm_kernel<BM, BN, WM, 128, BF16, EPI_SWIGLU, 128, DIRECT, NS, BK>),
-                       dim3(grid), block, 0, st, g, e);
-  } else {
-    hipLaunchKernelGGL((qkv_gemm_kernel<BM, BN, WM, 128, BF16, EPI_LINEAR, 128, DIRECT, NS, BK>),
-                       dim3(grid), block, 0, st, g, e);
-  }
-}
-
+// The linear fusions whose K the DMA path of linear_gemm.hip does not take (K
+// not a multiple of 64, or operands of 4 GiB and more): register-staged tiles.
 template <bool BF16>
-static void launch_linear(const QkvPlan& p, const GemmArgs& g, const QkvEpi& e, bool swiglu,
-                          int64_t wrows, hipStream_t st) {
-  const bool dma = g.k % 64 == 0 && g.lda % 8 == 0 && g.ldw % 8 == 0 && aligned16(g.a) &&
-                   aligned16(g.w) && g.m * g.lda * 2 < (int64_t(1) << 32) &&
-                   wrows * g.ldw * 2 < (int64_t(1) << 32);
-  if (!dma) {
-    launch_linear_tile<128, 128, 32, 2, 64, BF16, false>(g, e, swiglu, st);
-    return;
-  }
-  switch (p.tile) {
-    case 2: launch_linear_tile<256, 256, 64, 2, 64, BF16, true>(g, e, swiglu, st); break;
-    case 3: launch_linear_tile<128, 256, 32, 2, 64, BF16, true>(g, e, swiglu, st); break;
-    case 1: launch_linear_tile<128, 256, 64, 3, 32, BF16, true>(g, e, swiglu, st); break;
-    default: launch_linear_tile<128, 128, 32, 4, 32, BF16, true>(g, e, swiglu, st); break;
-  }
+static void launch_linear(const GemmArgs& g, const QkvEpi& e, bool swiglu, hipStream_t st) {
+  const dim3 grid(static_cast<unsigned>(cdiv(g.m, 128) * cdiv(g.n, swiglu ? 64 : 128)));
+  if (swiglu)
+    hipLaunchKernelGGL((qkv_gemm_kernel<128, 128, 32, 128, BF16, EPI_SWIGLU, 128, false, 2, 64>), grid, dim3(256), 0,
+                       st, g, e);
+  else
+    hipLaunchKernelGGL((qkv_gemm_kernel<128, 128, 32, 128, BF16, EPI_LINEAR, 128, false, 2, 64>), grid, dim3(256), 0,
+                       st, g, e);
 }
 
 template <bool BF16, bool DIRECT>
@@ -3366,7 +3330,10 @@ extern "C" int64_t bfa_linear_workspace_size(int64_t tokens, int64_t k, int64_t 
   if (tokens <= 0 || n <= 0) return 0;
   const int64_t nw = mode == BFA_LINEAR_SILU_AND_MUL ? 2 * n : n;
   const QkvPlan p = make_plan(tokens, nw, k, 0);
-  return p.decode ? p.part_bytes : 0;  // prefill tiles finish in their epilogue
+  if (p.decode) return p.part_bytes;
+  // above 64 tokens: the fp32 partials of the tiles that are split over K; a
+  // caller without that workspace gets the plan without a split
+  return k % 64 == 0 ? linear_plan(tokens, n, k, mode == BFA_LINEAR_SILU_AND_MUL, true).part_bytes : 0;
 }
 
 extern "C" int bfa_linear(const void* x, int dtype, int64_t tokens, int64_t k, int64_t x_stride,
@@ -3435,6 +3402,20 @@ extern "C" int bfa_linear(const void* x, int dtype, int64_t tokens, int64_t k, i
     }
     return check_launch(what);
   }
-  if (bf16) launch_linear<true>(p, g, e, swiglu, nw, st); else launch_linear<false>(p, g, e, swiglu, nw, st);
+  if (k % 64 == 0 && tokens * x_stride * 2 < (int64_t(1) << 32) && nw * w_stride * 2 < (int64_t(1) << 32)) {
+    LinArgs q{};
+    q.a = g.a; q.w = g.w; q.m = tokens; q.n = n; q.k = k; q.lda = x_stride; q.ldw = w_stride;
+    q.bias = bias; q.bias_dt = bias_dtype; q.res = residual; q.res_dt = residual_dtype; q.ldr = residual_stride;
+    q.out = out; q.ldo = out_stride;
+    q.proj_dt = proj_dtype; q.mid_dt = sum_dtype; q.out_dt = out_dtype;
+    q.vec = e.vec; q.swiglu = swiglu ? 1 : 0;
+    LinPlan lp = linear_plan(tokens, n, k, swiglu, true);
+    if (lp.part_bytes > 0 && (workspace_bytes < lp.part_bytes || !workspace || !aligned16(workspace)))
+      lp = linear_plan(tokens, n, k, swiglu, false);
+    q.part = static_cast<float*>(workspace);
+    launch_linear_gemm(lp, q, dtype, st);
+    return check_launch(what);
+  }
+  if (bf16) launch_linear<true>(g, e, swiglu, st); else launch_linear<false>(g, e, swiglu, st);
   return check_launch(what);
 }

@@ -78,7 +78,9 @@ const char* bfa_last_error(void);
                                         the 256x256 tile, 0 for the others) */
 #define BFA_TUNE_DECODE_GEMV 12      /* BFA_DECODE_GEMV: 0 = never the one-launch decode kernel
                                         (1-8 tokens without q/k norm) */
-#define BFA_TUNE_COUNT 13
+#define BFA_TUNE_LINEAR_TILE 13      /* BFA_LINEAR_TILE: tile id of the linear GEMM (65+ tokens) */
+#define BFA_TUNE_LINEAR_SPLITS 14    /* BFA_LINEAR_SPLITS: its K splits */
+#define BFA_TUNE_COUNT 15
 int bfa_set_tuning(int key, int value);
 int bfa_get_tuning(int key);
 
@@ -471,7 +473,8 @@ int bfa_cascade_attention(const void* query, int dtype, int64_t num_tokens, int6
  * x [tokens, k] and weight (row strides x_stride / w_stride, multiples of 8,
  * 16-byte aligned) share a dtype, bf16 or fp16; k a multiple of 16.  out
  * [tokens, n] (row stride out_stride).  workspace: bfa_linear_workspace_size
- * bytes (split-K partials for up to 64 tokens; 0 above). */
+ * bytes (split-K partials; above 64 tokens a smaller workspace, or none, is
+ * accepted too and leaves every tile whole). */
 enum { BFA_LINEAR_PLAIN = 0, BFA_LINEAR_SILU_AND_MUL = 1 };
 int64_t bfa_linear_workspace_size(int64_t tokens, int64_t k, int64_t n, int mode);
 int bfa_linear(const void* x, int dtype, int64_t tokens, int64_t k, int64_t x_stride,
