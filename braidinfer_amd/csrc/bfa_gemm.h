@@ -1,4 +1,4 @@
-// Main loop of the 16x16x32-MFMA GEMMs on 16-bit operands (linear_gemm.hip):
+// Main loop of the 16x16x32-MFMA GEMMs on 16-bit operands (linear_gemm.hip, qkv_prefill.hip):
 // acc = W X^T of one BM x BN tile over a range of 64-deep K stages, both
 // operands through a ring of LDS stages filled by DMA.
 #pragma once

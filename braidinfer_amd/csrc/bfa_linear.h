@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "bfa_gemm_plan.h"
+
 namespace bfa {
 
 // y = out_dt(mid_dt(proj_dt(x W^T + bias) + res)), or with swiglu
@@ -27,17 +29,9 @@ struct LinArgs {
   int tiles_m, tiles_n, full, splits, kt;
 };
 
-struct LinPlan {
-  int tile;
-  int full;    // tiles taken whole; the others are split over K
-  int splits;
-  int64_t tiles_m, tiles_n;
-  int64_t part_bytes;
-};
-
 // The plan for m tokens and n output columns (2 n weight rows with swiglu);
 // split = false: without split K, so without a workspace.
-LinPlan linear_plan(int64_t m, int64_t n, int64_t k, bool swiglu, bool split);
-void launch_linear_gemm(const LinPlan& p, LinArgs q, int dt, hipStream_t st);
+GemmPlan linear_plan(int64_t m, int64_t n, int64_t k, bool swiglu, bool split);
+void launch_linear_gemm(const GemmPlan& p, LinArgs q, int dt, hipStream_t st);
 
 }  // namespace bfa

@@ -4,7 +4,7 @@
 // What bounds it: from about a thousand tokens the matrix cores (under their
 // load the chip is power limited), below that the weight stream and the number
 // of CUs that have a tile.  A workgroup of RW x CW waves owns a BM x BN tile
-// and runs the ring of bfa_gemm.h.  The tile sizes differ in how well they fill
+// and runs the ring of bfa_gemm.h.  The tile sizes (bfa_gemm_plan.h) differ in how well they fill
 // the 256 CUs, which decides more than the loop does (Llama-3-8B, 300 tokens:
 // gate_up on 128 x 256 tiles is 336 tiles, two rounds of which the second is
 // nearly empty; on 160 x 256 it is one round of 224).  What whole rounds of
@@ -192,104 +192,34 @@ __global__ __launch_bounds__(256) void linear_reduce_kernel(LinArgs q, int ma, i
 // ------------------------------------------------------------------- host
 namespace {
 
-// The tiles, and a stage's time on a full chip (BM x BN x 64, 256 workgroups,
-// measured at 6000 tokens with K = 4096 and 14336): the planner compares tiles
-// by rounds x stages x this.  The wide tiles do more per LDS byte (0.95 us for
-// 128 x 256 against 1.55 for twice the work), the small ones fill a short grid.
-struct LinTile {
-  int ma, rw, cw;
-  double stage_us;
-};
-constexpr LinTile kTiles[] = {
-    {8, 2, 4, 1.55},  // 0: 256 x 256, 2 stages
-    {6, 2, 4, 1.30},  // 1: 192 x 256, 2
-    {5, 2, 4, 1.12},  // 2: 160 x 256, 3
-    {4, 2, 4, 0.95},  // 3: 128 x 256, 3
-    {4, 4, 2, 0.96},  // 4: 256 x 128, 3
-    {3, 4, 2, 0.75},  // 5: 192 x 128, 4
-    {2, 4, 2, 0.58},  // 6: 128 x 128, 5
-    {1, 4, 2, 0.38},  // 7:  64 x 128, 6
-};
-constexpr int kNumTiles = static_cast<int>(sizeof(kTiles) / sizeof(kTiles[0]));
-
-template <int MA, int RW, int CW, int NS, int DT, bool SAME>
-void launch_tile(const LinArgs& q, hipStream_t st) {
-  const int rest = q.tiles_m * q.tiles_n - q.full;
-  const dim3 grid(static_cast<unsigned>(q.full + rest * q.splits)), block(RW * CW * 64);
-  if (q.swiglu) hipLaunchKernelGGL((linear_gemm_kernel<MA, RW, CW, NS, DT, SAME, true>), grid, block, 0, st, q);
-  else hipLaunchKernelGGL((linear_gemm_kernel<MA, RW, CW, NS, DT, SAME, false>), grid, block, 0, st, q);
-}
-
 template <int DT, bool SAME>
-void launch_form(const LinPlan& p, const LinArgs& q, hipStream_t st) {
-  switch (p.tile) {
-    case 0: launch_tile<8, 2, 4, 2, DT, SAME>(q, st); break;
-    case 1: launch_tile<6, 2, 4, 2, DT, SAME>(q, st); break;
-    case 2: launch_tile<5, 2, 4, 3, DT, SAME>(q, st); break;
-    case 3: launch_tile<4, 2, 4, 3, DT, SAME>(q, st); break;
-    case 4: launch_tile<4, 4, 2, 3, DT, SAME>(q, st); break;
-    case 5: launch_tile<3, 4, 2, 4, DT, SAME>(q, st); break;
-    case 6: launch_tile<2, 4, 2, 5, DT, SAME>(q, st); break;
-    default: launch_tile<1, 4, 2, 6, DT, SAME>(q, st); break;
-  }
+void launch_form(const GemmPlan& p, const LinArgs& q, hipStream_t st) {
   const int rest = q.tiles_m * q.tiles_n - q.full;
+  const dim3 grid(static_cast<unsigned>(q.full + rest * q.splits));
+  gemm_tile_dispatch(p.tile, [&](auto t) {
+    using S = decltype(t);
+    const dim3 block(S::RW * S::CW * 64);
+    if (q.swiglu) hipLaunchKernelGGL((linear_gemm_kernel<S::MA, S::RW, S::CW, S::NS, DT, SAME, true>), grid, block, 0, st, q);
+    else hipLaunchKernelGGL((linear_gemm_kernel<S::MA, S::RW, S::CW, S::NS, DT, SAME, false>), grid, block, 0, st, q);
+  });
   if (rest > 0) {
-    const LinTile& t = kTiles[p.tile];
+    const GemmTileInfo& t = kGemmTiles[p.tile];
     const int items = rest * t.rw * t.cw * t.ma;
-    const dim3 grid(static_cast<unsigned>(cdiv(items, 4)));
-    if (q.swiglu) hipLaunchKernelGGL((linear_reduce_kernel<DT, SAME, true>), grid, dim3(256), 0, st, q, t.ma, t.rw, t.cw, items);
-    else hipLaunchKernelGGL((linear_reduce_kernel<DT, SAME, false>), grid, dim3(256), 0, st, q, t.ma, t.rw, t.cw, items);
+    const dim3 rgrid(static_cast<unsigned>(cdiv(items, 4)));
+    if (q.swiglu) hipLaunchKernelGGL((linear_reduce_kernel<DT, SAME, true>), rgrid, dim3(256), 0, st, q, t.ma, t.rw, t.cw, items);
+    else hipLaunchKernelGGL((linear_reduce_kernel<DT, SAME, false>), rgrid, dim3(256), 0, st, q, t.ma, t.rw, t.cw, items);
   }
 }
 
 }  // namespace
 
-// Each tile is weighed with every tile whole and, where the last round is not
-// full, with that round's tiles split over K as often as the CUs allow: rounds
-// times (stages x stage_us + 4 us of fill and epilogue), and for split tiles the
-// second launch and the partials' round trip.  Overrides: BFA_TUNE_LINEAR_TILE,
-// BFA_TUNE_LINEAR_SPLITS.
-LinPlan linear_plan(int64_t m, int64_t n, int64_t k, bool swiglu, bool split) {
-  const int ot = tuning(BFA_TUNE_LINEAR_TILE), os = tuning(BFA_TUNE_LINEAR_SPLITS);
-  const int64_t kt = k / 64;
-  LinPlan best{};
-  double cost = 0;
-  for (int id = 0; id < kNumTiles; ++id) {
-    if (ot >= 0 && ot < kNumTiles && id != ot) continue;
-    const LinTile& t = kTiles[id];
-    LinPlan p{};
-    p.tile = id;
-    p.tiles_m = cdiv(m, 16 * t.ma * t.rw);
-    p.tiles_n = cdiv(n, (swiglu ? 32 : 64) * t.cw);
-    const int64_t tiles = p.tiles_m * p.tiles_n, rounds = tiles / 256, rest = tiles % 256;
-    p.full = static_cast<int>(tiles);
-    p.splits = 1;
-    double c = static_cast<double>(rounds + (rest > 0)) * (kt * t.stage_us + 4.0);
-    int64_t s = rest > 0 ? 256 / rest : 1;
-    if (os >= 1) s = os;
-    s = std::min<int64_t>(std::min<int64_t>(s, kt), 32);
-    if (split && rest > 0 && s > 1) {
-      const int64_t bytes = rest * s * t.rw * t.cw * t.ma * 4 * 64 * 16;
-      const double cs = static_cast<double>(rounds) * (kt * t.stage_us + 4.0) + cdiv(rest * s, 256) * (cdiv(kt, s) * t.stage_us + 4.0) +
-                        4.0 + static_cast<double>(bytes) / 3.0e6;
-      if (cs < c || os > 1) {
-        c = cs;
-        p.full = static_cast<int>(rounds * 256);
-        p.splits = static_cast<int>(s);
-        p.part_bytes = bytes;
-      }
-    }
-    if (best.splits == 0 || c < cost) {
-      best = p;
-      cost = c;
-    }
-  }
-  return best;
+GemmPlan linear_plan(int64_t m, int64_t n, int64_t k, bool swiglu, bool split) {
+  return gemm_plan(m, swiglu ? 2 * n : n, k, 4.0, split ? INT64_MAX : 0);
 }
 
-void launch_linear_gemm(const LinPlan& p, LinArgs q, int dt, hipStream_t st) {
-  q.tiles_m = static_cast<int>(p.tiles_m);
-  q.tiles_n = static_cast<int>(p.tiles_n);
+void launch_linear_gemm(const GemmPlan& p, LinArgs q, int dt, hipStream_t st) {
+  q.tiles_m = p.tiles_m;
+  q.tiles_n = p.tiles_n;
   q.full = p.full;
   q.splits = p.splits;
   q.kt = static_cast<int>(q.k / 64);

@@ -14,7 +14,9 @@
 // QKVParallelLinear (layers/linear.py:78-114).
 //
 // Kernels
-//  * qkv_gemm_kernel   prefill.  BMxBN tile per workgroup of 4 or 8 waves, each
+//  * qkv_prefill_kernel (qkv_prefill.hip)  prefill, head_dim 64 and 128, K a
+//    multiple of 64.
+//  * qkv_gemm_kernel   the other prefill shapes.  BMxBN tile per workgroup of 4 or 8 waves, each
 //    wave WMx128: v_mfma_f32_16x16x32_{bf16,f16} on the 64-deep DMA path,
 //    v_mfma_f32_32x32x16 on the 32-deep rings and the register-staged path;
 //    256x256 with 8 waves (two per SIMD) for large token counts.  Operand and weight K-slices move HBM ->
@@ -47,6 +49,7 @@
 #include "bfa_internal.h"
 #include "bfa_linear.h"
 #include "bfa_qkv.h"
+#include "bfa_qkv_prefill.h"
 
 namespace bfa {
 
@@ -95,15 +98,7 @@ __device__ __forceinline__ void store4_any(void* p, int dt, int64_t i, const flo
   }
 }
 
-// Branch-free forms for the GEMM epilogue, whose code is unrolled over every
-// row a lane owns: a rounding or store that dispatches on the dtype with
-// branches there grew the kernel past the instruction cache.  dt is uniform.
-__device__ __forceinline__ float round_sel(float v, int dt) {
-  const float rb = Elem<BFA_DTYPE_BF16>::round(v);
-  const float rh = Elem<BFA_DTYPE_F16>::round(v);
-  return dt == BFA_DTYPE_BF16 ? rb : (dt == BFA_DTYPE_F16 ? rh : v);
-}
-
+// (branch-free, as round_sel)
 __device__ __forceinline__ uint32_t pack2_sel(float lo, float hi, bool bf) {
   const uint32_t b = f32_to_bf16_bits(lo) | (static_cast<uint32_t>(f32_to_bf16_bits(hi)) << 16);
   const uint32_t h = f32_to_f16_bits(lo) | (static_cast<uint32_t>(f32_to_f16_bits(hi)) << 16);
@@ -121,23 +116,6 @@ __device__ __forceinline__ void store4_sel(void* p, int dt, int64_t i, const flo
         make_uint2(pack2_sel(v[0], v[1], bf), pack2_sel(v[2], v[3], bf));
   }
 }
-
-// Epilogue dtype forms of the GEMM kernel.  EDT_RT reads every rounding and
-// store dtype from QkvEpi at run time (the branch-free selects above: each
-// rounds both ways and picks one).  The fixed forms compile the dtypes in for
-// the two combinations the decoders run, so a rounding is one conversion:
-//   EDT_F32_BF16  fp32 projection, no q/k norm, RoPE in fp32, bf16 store
-//                 (the Llama chain: minimal_f32 -> rotary_emb -> .to(bf16))
-//   EDT_BF16      every rounding point bf16 (the Qwen3 chain, the bf16 linears)
-enum { EDT_RT = 0, EDT_F32_BF16 = 1, EDT_BF16 = 2 };
-template <int EDT> struct EpiDt { static constexpr int Q = -1, N = -1, A = -1, O = -1, M = -1; };
-template <> struct EpiDt<EDT_F32_BF16> {
-  static constexpr int Q = BFA_DTYPE_F32, N = -1, A = BFA_DTYPE_F32, O = BFA_DTYPE_BF16, M = -1;
-};
-template <> struct EpiDt<EDT_BF16> {
-  static constexpr int Q = BFA_DTYPE_BF16, N = BFA_DTYPE_BF16, A = BFA_DTYPE_BF16,
-                       O = BFA_DTYPE_BF16, M = BFA_DTYPE_BF16;
-};
 
 // Rounding to DT (compile time) or to the run-time dtype dt when DT < 0.
 template <int DT>
@@ -420,7 +398,7 @@ template <int EPI, int HD, int MB, int NB, int WM, int WN, int NW, int EDT, bool
 __device__ __forceinline__ void gemm_epilogue(ACC& acc, uint4* lds, const GemmArgs& g, const QkvEpi& e,
                                               int64_t m0, int64_t n0, int wid, int wm, int wn, int lane,
                                               const int64_t* praw) {
-  using DT = EpiDt<EDT>;
+  using DT = QkvDt<EDT>;
   constexpr bool A16 = sizeof(acc[0][0]) == sizeof(f32x4_t);  // 16x16 accumulator blocks
   constexpr int LDR = 136;
   constexpr bool EARLY_POS = EARLY;
@@ -1947,7 +1925,7 @@ __device__ __forceinline__ void wait_vm_dyn(int n) {
 // the weight already holds bf16(w * gamma) (bfa_fold_rmsnorm_weight).
 template <int MT, bool SA, int EDT, bool GIN = true>
 __global__ __launch_bounds__(256) void qkv_decode_pair_kernel(DecodeArgs d, QkvEpi e, int nch) {
-  using DT = EpiDt<EDT>;
+  using DT = QkvDt<EDT>;
   constexpr bool G = SA && GIN;         // gamma applied here
   constexpr int RX = PairRing<MT>::RX, RW = PairRing<MT>::RW;
   constexpr int ROWS = MT * 16;
@@ -2424,6 +2402,9 @@ struct QkvPlan {
   int nch;         // decode stream: 256-deep chunks per split of the deep-K form (0: not used)
   int64_t operand_bytes;
   int64_t part_bytes;
+  int64_t need_bytes;     // of which the call cannot do without
+  bool pre;               // prefill by qkv_prefill.hip, with `gemm`
+  GemmPlan gemm;
 };
 
 static int64_t align256(int64_t v) { return (v + 255) / 256 * 256; }
@@ -2493,6 +2474,7 @@ static QkvPlan make_plan(int64_t m, int64_t n, int64_t k, int64_t hd) {
     // 128 columns x 16 MT rows; otherwise row-major [splits, m, n]
     p.part_bytes = (p.stream && p.mt > 1) ? align256(p.splits * cdiv(n, 128) * 128 * p.mt * 16 * 4)
                                           : align256(p.splits * m * n * 4);
+    p.need_bytes = p.part_bytes;
   } else {
     p.decode = false;
     p.fused_epi = (hd == 32 || hd == 64 || hd == 128) && n % hd == 0;
@@ -2505,16 +2487,24 @@ static QkvPlan make_plan(int64_t m, int64_t n, int64_t k, int64_t hd) {
     else if (cdiv(m, 128) * cdiv(n, 256) >= 192) p.tile = 3;
     else p.tile = 128;
     // Under 128 tiles of 128x128 most CUs would idle, and each busy one is
-    // bound by its LDS traffic: for heads of up to 64 columns 128x64 tiles put
-    // twice the CUs on the product (TinyLlama, 512 tokens: 80 -> 160 tiles).
-    const bool narrow_ok = p.fused_epi && hd <= 64;
+    // bound by its LDS traffic: for heads of 32 columns 128x64 tiles put twice
+    // the CUs on the product.
+    const bool narrow_ok = p.fused_epi && hd == 32;
     if (p.tile == 128 && narrow_ok && cdiv(m, 128) * cdiv(n, 128) < 128) p.tile = 64;
     {
       const int v = tuning(BFA_TUNE_QKV_TILE);
       if ((v >= 1 && v <= 3) || v == 128 || (v == 64 && narrow_ok)) p.tile = v;
     }
     p.splits = 1;
-    p.part_bytes = p.fused_epi ? 0 : align256(m * n * 4);
+    p.need_bytes = p.fused_epi ? 0 : align256(m * n * 4);
+    p.part_bytes = p.need_bytes;
+    // head_dim 64 and 128 on the DMA path: qkv_prefill.hip (an optional
+    // workspace for its split tiles)
+    p.pre = p.fused_epi && hd >= 64 && k % 64 == 0;
+    if (p.pre) {
+      p.gemm = qkv_prefill_plan(m, n, k, p.operand_bytes, true);
+      p.part_bytes = align256(p.gemm.part_bytes);
+    }
   }
   return p;
 }
@@ -2619,26 +2609,8 @@ static int fused_edt(const QkvEpi& e) {
   if (e.qkv_dt == BFA_DTYPE_F32 && e.out_dt == BFA_DTYPE_BF16 && !norm) return EDT_F32_BF16;
   if (e.qkv_dt == BFA_DTYPE_BF16 && e.out_dt == BFA_DTYPE_BF16 && (!norm || e.norm_dt == BFA_DTYPE_BF16))
     return EDT_BF16;
+  if (e.qkv_dt == BFA_DTYPE_F32 && e.out_dt == BFA_DTYPE_F16 && !norm) return EDT_F32_F16;
   return EDT_RT;
-}
-
-template <int BM, int BN, int WM, int NS, int BK, bool BF16, bool DIRECT, int HD>
-static void launch_fused_edt(unsigned grid, dim3 block, int edt, const GemmArgs& g, const QkvEpi& e,
-                             hipStream_t st) {
-  if constexpr (BF16 && DIRECT && HD >= 64) {
-    if (edt == EDT_F32_BF16) {
-      hipLaunchKernelGGL((qkv_gemm_kernel<BM, BN, WM, 128, BF16, EPI_FUSED, HD, DIRECT, NS, BK, EDT_F32_BF16>),
-                         dim3(grid), block, 0, st, g, e);
-      return;
-    }
-    if (edt == EDT_BF16) {
-      hipLaunchKernelGGL((qkv_gemm_kernel<BM, BN, WM, 128, BF16, EPI_FUSED, HD, DIRECT, NS, BK, EDT_BF16>),
-                         dim3(grid), block, 0, st, g, e);
-      return;
-    }
-  }
-  hipLaunchKernelGGL((qkv_gemm_kernel<BM, BN, WM, 128, BF16, EPI_FUSED, HD, DIRECT, NS, BK>), dim3(grid),
-                     block, 0, st, g, e);
 }
 
 // Workgroups of a prefill GEMM launch: one per tile, or for the 256x256 tile
@@ -2661,38 +2633,34 @@ template <int BM, int BN, int WM, int NS, int BK, bool BF16, bool DIRECT>
 static void launch_prefill_tile(const QkvPlan& p, const GemmArgs& g, const QkvEpi& e, hipStream_t st) {
   const unsigned grid = persistent_grid(cdiv(g.m, BM) * cdiv(g.n, BN), BM == 256 && BN == 256);
   const dim3 block((BM / WM) * (BN / 128) * 64);
-  const int edt = fused_edt(e);
   if (!p.fused_epi) {
     hipLaunchKernelGGL((qkv_gemm_kernel<BM, BN, WM, 128, BF16, EPI_RAW, 128, DIRECT, NS, BK>), dim3(grid),
                        block, 0, st, g, e);
-  } else if (e.hd == 128) {
-    launch_fused_edt<BM, BN, WM, NS, BK, BF16, DIRECT, 128>(grid, block, edt, g, e, st);
-  } else if (e.hd == 64) {
-    launch_fused_edt<BM, BN, WM, NS, BK, BF16, DIRECT, 64>(grid, block, edt, g, e, st);
-  } else {
-    launch_fused_edt<BM, BN, WM, NS, BK, BF16, DIRECT, 32>(grid, block, edt, g, e, st);
+    return;
   }
+  if constexpr (!DIRECT) {
+    if (e.hd == 128) {
+      hipLaunchKernelGGL((qkv_gemm_kernel<BM, BN, WM, 128, BF16, EPI_FUSED, 128, DIRECT, NS, BK>), dim3(grid), block,
+                         0, st, g, e);
+      return;
+    }
+    if (e.hd == 64) {
+      hipLaunchKernelGGL((qkv_gemm_kernel<BM, BN, WM, 128, BF16, EPI_FUSED, 64, DIRECT, NS, BK>), dim3(grid), block,
+                         0, st, g, e);
+      return;
+    }
+  }
+  // head_dim 64 and 128 on the DMA path are qkv_prefill.hip's
+  hipLaunchKernelGGL((qkv_gemm_kernel<BM, BN, WM, 128, BF16, EPI_FUSED, 32, DIRECT, NS, BK>), dim3(grid), block, 0,
+                     st, g, e);
 }
 
 // 128x64 tile: four waves of 32x64, a ring of four 32-deep DMA stages, the
-// fused epilogue with 8 lanes per row (head_dim 32 or 64).
-template <bool BF16, int HD>
-static void launch_prefill_narrow_hd(const GemmArgs& g, const QkvEpi& e, hipStream_t st) {
+// fused epilogue with 8 lanes per row (head_dim 32).
+template <bool BF16>
+static void launch_prefill_narrow(const GemmArgs& g, const QkvEpi& e, hipStream_t st) {
   const dim3 grid(static_cast<unsigned>(cdiv(g.m, 128) * cdiv(g.n, 64))), block(256);
-  const int edt = fused_edt(e);
-  if constexpr (BF16) {
-    if (edt == EDT_F32_BF16) {
-      hipLaunchKernelGGL((qkv_gemm_kernel<128, 64, 32, 64, BF16, EPI_FUSED, HD, true, 4, 32, EDT_F32_BF16>), grid,
-                         block, 0, st, g, e);
-      return;
-    }
-    if (edt == EDT_BF16) {
-      hipLaunchKernelGGL((qkv_gemm_kernel<128, 64, 32, 64, BF16, EPI_FUSED, HD, true, 4, 32, EDT_BF16>), grid,
-                         block, 0, st, g, e);
-      return;
-    }
-  }
-  hipLaunchKernelGGL((qkv_gemm_kernel<128, 64, 32, 64, BF16, EPI_FUSED, HD, true, 4, 32>), grid, block, 0, st, g, e);
+  hipLaunchKernelGGL((qkv_gemm_kernel<128, 64, 32, 64, BF16, EPI_FUSED, 32, true, 4, 32>), grid, block, 0, st, g, e);
 }
 
 // The linear fusions whose K the DMA path of linear_gemm.hip does not take (K
@@ -2716,8 +2684,7 @@ static void launch_prefill_t(const QkvPlan& p, const GemmArgs& g, const QkvEpi& 
       case 3: launch_prefill_tile<128, 256, 32, 2, 64, BF16, true>(p, g, e, st); break;
       case 1: launch_prefill_tile<128, 256, 64, 3, 32, BF16, true>(p, g, e, st); break;
       case 64:
-        if (e.hd == 64) launch_prefill_narrow_hd<BF16, 64>(g, e, st);
-        else launch_prefill_narrow_hd<BF16, 32>(g, e, st);
+        launch_prefill_narrow<BF16>(g, e, st);
         break;
       default: launch_prefill_tile<128, 128, 32, 4, 32, BF16, true>(p, g, e, st); break;
     }
@@ -2866,10 +2833,10 @@ static int qkv_projection_impl(const void* operand, int64_t lda, const OperandFo
               "%s: output rows must be 16-byte aligned", what);
   BFA_REQUIRE(row_scale == nullptr || (!p.decode && p.fused_epi), "%s: row scales need the prefill epilogue",
               what);
-  BFA_REQUIRE(part_workspace_bytes >= p.part_bytes && (p.part_bytes == 0 || part_workspace),
+  BFA_REQUIRE(part_workspace_bytes >= p.need_bytes && (p.need_bytes == 0 || part_workspace),
               "%s: workspace too small (%lld < %lld bytes)", what, (long long)part_workspace_bytes,
-              (long long)p.part_bytes);
-  BFA_REQUIRE(p.part_bytes == 0 || aligned16(part_workspace), "%s: workspace must be 16-byte aligned",
+              (long long)p.need_bytes);
+  BFA_REQUIRE(p.need_bytes == 0 || aligned16(part_workspace), "%s: workspace must be 16-byte aligned",
               what);
 
   QkvEpi e{};
@@ -2967,6 +2934,15 @@ static int qkv_projection_impl(const void* operand, int64_t lda, const OperandFo
   g.w = static_cast<const uint16_t*>(qkv_weight);
   g.m = tokens; g.n = qkv_dim; g.k = hidden; g.lda = lda; g.ldw = w_stride;
   g.raw = part;
+  if (p.pre && lda % 8 == 0 && tokens * lda * 2 < (int64_t(1) << 32) && qkv_dim * w_stride * 2 < (int64_t(1) << 32)) {
+    QkvPrefillArgs q{};
+    q.a = g.a; q.w = g.w; q.m = tokens; q.k = hidden; q.lda = lda; q.ldw = w_stride;
+    q.part = part;
+    const bool fits = p.gemm.part_bytes == 0 ||
+                      (part && aligned16(part) && part_workspace_bytes >= p.gemm.part_bytes);
+    launch_qkv_prefill(fits ? p.gemm : qkv_prefill_plan(tokens, qkv_dim, hidden, 0, false), q, e, w_dtype, fused_edt(e), st);
+    return check_launch(what);
+  }
   if (bf16) launch_prefill<true>(p, g, e, st); else launch_prefill<false>(p, g, e, st);
   int rc = check_launch(what);
   if (rc != BFA_OK || p.fused_epi) return rc;
@@ -3006,9 +2982,9 @@ static int fused_impl(const void* x, int x_dtype, int64_t tokens, int64_t hidden
   const int64_t heads = num_q_heads + 2 * num_kv_heads;
   BFA_REQUIRE(heads > 0 && qkv_dim % heads == 0, "%s: bad head geometry", what);
   const QkvPlan p = make_plan(tokens, qkv_dim, hidden, qkv_dim / heads);
-  BFA_REQUIRE(workspace && workspace_bytes >= p.operand_bytes + p.part_bytes && aligned16(workspace),
+  BFA_REQUIRE(workspace && workspace_bytes >= p.operand_bytes + p.need_bytes && aligned16(workspace),
               "%s: workspace too small (%lld < %lld bytes)", what, (long long)workspace_bytes,
-              (long long)(p.operand_bytes + p.part_bytes));
+              (long long)(p.operand_bytes + p.need_bytes));
   char* ws = static_cast<char*>(workspace);
   // Up to 16 decode tokens whose x is already in the weight dtype: the
   // weight-streaming kernel normalises its own K slice, one launch fewer.  One
@@ -3145,16 +3121,16 @@ extern "C" int bfa_fused_rmsnorm_qkv_append(
   if (rc != BFA_OK || tokens == 0) return rc;
   const int64_t heads = num_q_heads + 2 * num_kv_heads;
   BFA_REQUIRE(heads > 0 && qkv_dim % heads == 0, "%s: bad head geometry", what);
-  const int64_t fsize = bfa_fused_rmsnorm_qkv_workspace_size(tokens, hidden, qkv_dim, qkv_dim / heads);
-  BFA_REQUIRE(workspace && aligned16(workspace) && workspace_bytes >= fsize + align256(tokens * 8),
-              "%s: workspace too small (%lld < %lld bytes)", what, (long long)workspace_bytes,
-              (long long)(fsize + align256(tokens * 8)));
+  const QkvPlan p = make_plan(tokens, qkv_dim, hidden, qkv_dim / heads);
+  const int64_t need = p.operand_bytes + p.need_bytes + align256(tokens * 8);
+  BFA_REQUIRE(workspace && aligned16(workspace) && workspace_bytes >= need,
+              "%s: workspace too small (%lld < %lld bytes)", what, (long long)workspace_bytes, (long long)need);
   // the prefill GEMM with the fused epilogue resolves the slots itself; every
   // other path reads them from the workspace tail, filled by a small kernel
-  const QkvPlan p = make_plan(tokens, qkv_dim, hidden, qkv_dim / heads);
+  const int64_t fsize = workspace_bytes - align256(tokens * 8);
   int64_t* slot_off = nullptr;
   if (p.decode || !p.fused_epi) {
-    slot_off = reinterpret_cast<int64_t*>(static_cast<char*>(workspace) + fsize);
+    slot_off = reinterpret_cast<int64_t*>(static_cast<char*>(workspace) + p.operand_bytes + p.need_bytes);
     launch_kv_slots(a, tokens, slot_off, as_stream(stream));
     rc = check_launch(what);
     if (rc != BFA_OK) return rc;
@@ -3209,8 +3185,8 @@ extern "C" int bfa_fused_rmsnorm_qkv_folded(
     return set_error(BFA_ERR_UNSUPPORTED,
                      "%s: the prefill epilogue (more than 64 tokens, head_dim 32, 64 or 128) or the "
                      "column-pair decode shapes (17-64 bf16 tokens) only", what);
-  const int64_t fsize = p.operand_bytes + p.part_bytes;
-  const int64_t need = fsize + (layer_cache && p.decode ? align256(tokens * 8) : 0);
+  const int64_t need = p.operand_bytes + p.need_bytes + (layer_cache && p.decode ? align256(tokens * 8) : 0);
+  const int64_t fsize = p.decode ? p.operand_bytes + p.need_bytes : workspace_bytes;
   BFA_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace),
               "%s: workspace too small (%lld < %lld bytes)", what, (long long)workspace_bytes, (long long)need);
   char* ws = static_cast<char*>(workspace);
@@ -3308,7 +3284,8 @@ extern "C" int bfa_fused_rmsnorm_qkv_noalloc(
   BFA_REQUIRE(tokens > 0 && hidden > 0 && qkv_dim > 0, "%s: bad geometry", what);
   const int64_t heads = num_q_heads + 2 * num_kv_heads;
   BFA_REQUIRE(num_q_heads > 0 && num_kv_heads > 0 && qkv_dim % heads == 0, "%s: bad head geometry", what);
-  const int64_t need = bfa_fused_rmsnorm_qkv_workspace_size(tokens, hidden, qkv_dim, qkv_dim / heads);
+  const QkvPlan p = make_plan(tokens, qkv_dim, hidden, qkv_dim / heads);
+  const int64_t need = p.operand_bytes + p.need_bytes;
   BFA_REQUIRE(need <= BFA_NOALLOC_SCRATCH_BYTES,
               "%s: %lld tokens x hidden %lld x qkv_dim %lld need %lld bytes of scratch, more than the "
               "%lld this entry point holds; call bfa_fused_rmsnorm_qkv with a workspace",
@@ -3409,7 +3386,7 @@ extern "C" int bfa_linear(const void* x, int dtype, int64_t tokens, int64_t k, i
     q.out = out; q.ldo = out_stride;
     q.proj_dt = proj_dtype; q.mid_dt = sum_dtype; q.out_dt = out_dtype;
     q.vec = e.vec; q.swiglu = swiglu ? 1 : 0;
-    LinPlan lp = linear_plan(tokens, n, k, swiglu, true);
+    GemmPlan lp = linear_plan(tokens, n, k, swiglu, true);
     if (lp.part_bytes > 0 && (workspace_bytes < lp.part_bytes || !workspace || !aligned16(workspace)))
       lp = linear_plan(tokens, n, k, swiglu, false);
     q.part = static_cast<float*>(workspace);

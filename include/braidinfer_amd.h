@@ -78,8 +78,8 @@ const char* bfa_last_error(void);
                                         the 256x256 tile, 0 for the others) */
 #define BFA_TUNE_DECODE_GEMV 12      /* BFA_DECODE_GEMV: 0 = never the one-launch decode kernel
                                         (1-8 tokens without q/k norm) */
-#define BFA_TUNE_LINEAR_TILE 13      /* BFA_LINEAR_TILE: tile id of the linear GEMM (65+ tokens) */
-#define BFA_TUNE_LINEAR_SPLITS 14    /* BFA_LINEAR_SPLITS: its K splits */
+#define BFA_TUNE_GEMM_TILE 13      /* BFA_GEMM_TILE: tile id of the GEMMs above 64 tokens (0-7) */
+#define BFA_TUNE_GEMM_SPLITS 14    /* BFA_GEMM_SPLITS: its K splits */
 #define BFA_TUNE_COUNT 15
 int bfa_set_tuning(int key, int value);
 int bfa_get_tuning(int key);

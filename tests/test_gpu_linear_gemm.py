@@ -25,8 +25,8 @@ TILE_TOKENS = (256, 192, 160, 128, 256, 192, 128, 64)
 def test_tiles(tuning, tile, splits, edge):
     """One token short of and one past a whole row of tiles; 4 K stages over 3
     splits (1, 1 and 2 stages, fewer than the ring holds)."""
-    tuning("LINEAR_TILE", tile)
-    tuning("LINEAR_SPLITS", splits)
+    tuning("GEMM_TILE", tile)
+    tuning("GEMM_SPLITS", splits)
     t, k, n = max(2 * TILE_TOKENS[tile] + edge, 65), 256, 392
     g = gen(4000 + tile)
     x, w, r = randn(g, t, k), randn(g, n, k, std=0.03), randn(g, t, n, std=2.0)
@@ -46,7 +46,7 @@ def test_tiles(tuning, tile, splits, edge):
 def test_general_forms(tuning, splits):
     """n not a multiple of 8, a bias in fp32, fp16 operands, and the fp32 -> fp16
     rounding of the attention output."""
-    tuning("LINEAR_SPLITS", splits)
+    tuning("GEMM_SPLITS", splits)
     g = gen(4100)
     t, k, n = 77, 192, 203
     x, w, b = randn(g, t, k), randn(g, n, k, std=0.03), torch.randn(n, generator=g)
