@@ -165,8 +165,12 @@ constexpr int CAS_VP = 32 + 8;      // V^T row pitch (bf16): 80 bytes
 // two floats rounded to the 16-bit type, packed low | high << 16
 template <bool BF16>
 __device__ __forceinline__ uint32_t pack_pair(float lo, float hi) {
-  using E = Elem<BF16 ? BFA_DTYPE_BF16 : BFA_DTYPE_F16>;
-  return static_cast<uint32_t>(E::from_f32(lo)) | (static_cast<uint32_t>(E::from_f32(hi)) << 16);
+  if constexpr (BF16) {
+    return pack_bf16x2(lo, hi);  // one conversion for both
+  } else {
+    using E = Elem<BFA_DTYPE_F16>;
+    return static_cast<uint32_t>(E::from_f32(lo)) | (static_cast<uint32_t>(E::from_f32(hi)) << 16);
+  }
 }
 
 // N consecutive 16-bit elements (N = 2, 4 or 8: 4, 8 or 16 bytes, aligned to
@@ -646,8 +650,25 @@ __device__ __forceinline__ int kslot(int r, int gr) {
   else return gr ^ ((r >> 1) & 7);
 }
 
-template <bool BF16, int D>
-__global__ __launch_bounds__(256) void cascade_flat_kernel(CasArgs a, FlatArgs f) {
+// One wave takes RB blocks of 16 query rows, so a K or V^T fragment read from the
+// LDS feeds RB MFMAs.  With RB = 1 the loop is bound by those reads (32 KiB per
+// wave and tile, 2000 LDS cycles per CU against 1024 of MFMA) and by the softmax's
+// VALU work; RB = 2 halves the first, and per score the second is a maximum, one
+// multiply-add, the exponential, the sum and half a conversion:
+//   * tiles whose keys every row of the wave may see skip the masking (one
+//     compare per lane; a tile with the unused slots of a page, or at the causal
+//     edge, takes it);
+//   * the scale goes into the exponential's argument.
+// The running maximum follows every larger score: letting it lag by up to 2^8
+// saved rescalings (124 against 129 us for the call below) but rounded the largest p, exactly 1
+// otherwise, and the error against 64 bits rose from 0.0069 to 0.0070.
+// Qwen3 shape, 1000 queries over 9000 keys: the call 197 -> 129 us (this kernel
+// 176 -> 104 us, 670 TFLOP/s of attended pairs); Llama-3-8B 333 -> 212 us.
+// Moving the exponentials of one tile between the MFMAs of the next tile's scores
+// (two score sets) was slower, 126 against 123 us, and so were raised wave
+// priorities around the products (126 against 124 us).
+template <bool BF16, int D, int RB>
+__global__ __launch_bounds__(256, 2) void cascade_flat_kernel(CasArgs a, FlatArgs f) {
   // K tile: 64 rows of D * 2 bytes (GK granules, slots by kslot); V^T tile: D
   // rows of 128 bytes, granule G of row r at slot G ^ ((r / 2) & 7).
   constexpr int GK = D / 8, QJ = D / 32, OJ = D / 16;
@@ -660,27 +681,52 @@ __global__ __launch_bounds__(256) void cascade_flat_kernel(CasArgs a, FlatArgs f
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t g = blockIdx.y;
   const int64_t rows = a.tokens * a.group;
-  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * 64 + wid * 16;
+  const int64_t row0 = (static_cast<int64_t>(blockIdx.x) * 4 + wid) * (16 * RB);
   const int64_t tiles = f.npad / CAS_FT;
   const int64_t tl0 = static_cast<int64_t>(blockIdx.z) * f.tiles_per_split;
   const int64_t tl1 = min(tl0 + f.tiles_per_split, tiles);
 
-  uint4 qf[QJ];
-  {
-    const int64_t r = min(row0 + (lane & 15), rows - 1);
+  // base-2 scores; a negative scale turns the queries' signs instead
+  const float sl2 = fabsf(a.scale * 1.4426950408889634f);
+  const uint32_t flip = a.scale < 0.f ? 0x80008000u : 0u;
+  uint4 qf[RB][QJ];
+  int32_t qp[RB];             // query position, in the key positions' 32 bits
+  int32_t qmin = INT32_MAX, qmax = INT32_MIN;  // over the wave's rows
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    const int64_t r = min(row0 + 16 * rb + (lane & 15), rows - 1);
     const int64_t t = r / a.group, hh = g * a.group + (r - t * a.group);
     const uint16_t* qrow = a.q + t * a.q_st + hh * a.q_sh;
 #pragma unroll
-    for (int j = 0; j < QJ; ++j) qf[j] = *reinterpret_cast<const uint4*>(qrow + 32 * j + 8 * (lane >> 4));
+    for (int j = 0; j < QJ; ++j) {
+      const uint4 v = *reinterpret_cast<const uint4*>(qrow + 32 * j + 8 * (lane >> 4));
+      qf[rb][j] = make_uint4(v.x ^ flip, v.y ^ flip, v.z ^ flip, v.w ^ flip);
+    }
+    int64_t pos = INT32_MAX - 1;  // without a causal mask every key is seen
+    if (a.causal)
+      pos = a.qpos_i64 ? static_cast<const int64_t*>(a.qpos)[t] : static_cast<const int32_t*>(a.qpos)[t];
+    qp[rb] = static_cast<int32_t>(max(min(pos, static_cast<int64_t>(INT32_MAX - 1)), static_cast<int64_t>(INT32_MIN)));
   }
-  const int64_t qt = min(row0 + (lane & 15), rows - 1) / a.group;
-  const int64_t qp = a.qpos_i64 ? static_cast<const int64_t*>(a.qpos)[qt]
-                                : static_cast<const int32_t*>(a.qpos)[qt];
-  const float sl2 = a.scale * 1.4426950408889634f;
-  float m = -INFINITY, l = 0.f;
-  cas_f32x4_t o[OJ];
 #pragma unroll
-  for (int j = 0; j < OJ; ++j) o[j] = cas_f32x4_t{};
+  for (int rb = 0; rb < RB; ++rb) {
+    int32_t lo = qp[rb], hi = qp[rb];
+#pragma unroll
+    for (int d = 1; d < 16; d *= 2) {
+      lo = min(lo, __shfl_xor(lo, d));
+      hi = max(hi, __shfl_xor(hi, d));
+    }
+    qmin = min(qmin, lo);
+    qmax = max(qmax, hi);
+  }
+  float m[RB], l[RB];
+  cas_f32x4_t o[RB][OJ];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    m[rb] = -INFINITY;
+    l[rb] = 0.f;
+#pragma unroll
+    for (int j = 0; j < OJ; ++j) o[rb][j] = cas_f32x4_t{};
+  }
 
   // DMA roles per wave: K copy i moves rows (64 / GK) (4 i + wid) .. (lane: row +
   // lane / GK, slot lane % GK); V^T copy i moves rows 8 (4 i + wid) .. +7 (lane:
@@ -700,118 +746,150 @@ __global__ __launch_bounds__(256) void cascade_flat_kernel(CasArgs a, FlatArgs f
   const uint16_t* kbase = f.kf + g * f.npad * D;
   const uint16_t* vbase = f.vt + g * D * f.npad;
   const uint32_t kl = lds_addr(kbuf), vl = lds_addr(vbuf);
-  auto issue = [&](int64_t t, int b) {
+  auto issue_k = [&](int64_t t, int b) {
     const uint16_t* kt = kbase + t * CAS_FT * D;
-    const uint16_t* vt = vbase + t * CAS_FT;
 #pragma unroll
     for (int i = 0; i < KC; ++i) dma16(kt, koff[i], kl + b * (CAS_FT * GK * 16) + (4 * i + wid) * 1024);
+  };
+  auto issue_v = [&](int64_t t, int b) {
+    const uint16_t* vt = vbase + t * CAS_FT;
 #pragma unroll
     for (int i = 0; i < VC; ++i) dma16(vt, voff[i], vl + b * (D * 128) + (4 * i + wid) * 1024);
   };
-  // key positions of this lane's scores: slots 16 b + 4 (lane / 16) .. +3
-  auto load_kp = [&](int64_t t, int4 (&kp)[4]) {
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-      kp[b] = *reinterpret_cast<const int4*>(f.kpos + t * CAS_FT + 16 * b + 4 * (lane >> 4));
-  };
 
   if (tl0 < tl1) {
-    int4 kp[4];
-    issue(tl0, 0);
-    load_kp(tl0, kp);
-    wait_vmem();
-    __syncthreads();
-    for (int64_t t = tl0; t < tl1; ++t) {
-      const int b = static_cast<int>((t - tl0) & 1);
-      int4 kpn[4] = {kp[0], kp[1], kp[2], kp[3]};
-      if (t + 1 < tl1) {  // the next tile flies during this one's matrix work
-        issue(t + 1, b ^ 1);
-        load_kp(t + 1, kpn);
-      }
-      // S^T = K Q^T, 4 blocks of 16 keys: sacc[c][i] is the score of key slot
-      // 16 c + 4 (lane / 16) + i for query lane % 16
-      const uint4* kb = kbuf[b];
-      cas_f32x4_t sacc[4];
+    cas_f32x4_t sc[RB][4];  // the current tile's scores
+    // S^T = K Q^T, 4 blocks of 16 keys: s[rb][c][i] is the score of key slot
+    // 16 c + 4 (lane / 16) + i for query lane % 16 of block rb
+    auto scores = [&](const uint4* kb, cas_f32x4_t (&s)[RB][4]) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        sacc[c] = cas_f32x4_t{};
-        const int kr = 16 * c + (lane & 15);
+      for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int j = 0; j < QJ; ++j)
-          sacc[c] = mfma16x32<BF16>(kb[kr * GK + kslot<D>(kr, 4 * j + (lane >> 4))], qf[j], sacc[c]);
-      }
-      float p[4][4];
-      float mx = -INFINITY;
+        for (int rb = 0; rb < RB; ++rb) s[rb][c] = cas_f32x4_t{};
+      // (the key blocks inside: an MFMA's sum is next used 4 RB MFMAs later)
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const int kq[4] = {kp[c].x, kp[c].y, kp[c].z, kp[c].w};
+      for (int j = 0; j < QJ; ++j)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const bool use = kq[i] != INT32_MAX && (!a.causal || kq[i] <= qp);
-          p[c][i] = use ? sacc[c][i] * sl2 : -INFINITY;
-          mx = fmaxf(mx, p[c][i]);
+        for (int c = 0; c < 4; ++c) {
+          const int kr = 16 * c + (lane & 15);
+          const uint4 kf = kb[kr * GK + kslot<D>(kr, 4 * j + (lane >> 4))];
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb) s[rb][c] = mfma16x32<BF16>(kf, qf[rb][j], s[rb][c]);
         }
-      }
-      mx = lanes4_max(mx);
-      const float m_new = fmaxf(m, mx);
-      const float mref = m_new == -INFINITY ? 0.f : m_new;
-      const float alpha = __builtin_amdgcn_exp2f(m - mref);
-      float rs = 0.f;
+    };
+    auto mask = [&](int32_t kp, cas_f32x4_t (&s)[RB][4]) {
+      if (!__any(kp > qmin)) return;
 #pragma unroll
       for (int c = 0; c < 4; ++c)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          p[c][i] = __builtin_amdgcn_exp2f(p[c][i] - mref);
-          rs += p[c][i];
+          const int32_t kq = __shfl(kp, 16 * c + 4 * (lane >> 4) + i);
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb) s[rb][c][i] = kq > qp[rb] ? -INFINITY : s[rb][c][i];
         }
-      rs = lanes4_sum(rs);
-      l = l * alpha + rs;
-      m = m_new;
-      if (__any(alpha != 1.0f)) {
+    };
+    auto tile_max = [&](const cas_f32x4_t (&s)[4]) {
+      float mx = -INFINITY;
 #pragma unroll
-        for (int j = 0; j < OJ; ++j) o[j] *= alpha;
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[c][i]);
+      return mx;
+    };
+    auto new_max = [&](int rb, float mx) {
+      mx = lanes4_max(mx) * sl2;
+      if (!__any(mx > m[rb])) return;
+      const float m_new = fmaxf(m[rb], mx);
+      const float alpha = __builtin_amdgcn_exp2f(m[rb] - (m_new == -INFINITY ? 0.f : m_new));
+      m[rb] = m_new;
+      l[rb] *= alpha;
+#pragma unroll
+      for (int j = 0; j < OJ; ++j) o[rb][j] *= alpha;
+    };
+    // waits for every copy of this wave, and for `kp`'s load, which the compiler
+    // then holds complete: its own wait for it would also wait for copies issued
+    // later
+    auto arrive = [&](int32_t& kp) {
+      asm volatile("s_waitcnt vmcnt(0)" : "+v"(kp) : : "memory");
+      __syncthreads();
+    };
+    int32_t kp = f.kpos[tl0 * CAS_FT + lane];  // key position of slot `lane` of a tile
+    issue_k(tl0, 0);
+    issue_v(tl0, 0);
+    arrive(kp);
+    for (int64_t t = tl0; t < tl1; ++t) {
+      const int b = static_cast<int>((t - tl0) & 1);
+      int32_t kpn = f.kpos[min(t + 1, tl1 - 1) * CAS_FT + lane];
+      if (t + 1 < tl1) {  // the next tile flies during this one's matrix work
+        issue_k(t + 1, b ^ 1);
+        issue_v(t + 1, b ^ 1);
       }
-      // O^T += V^T P^T over the two groups of 32 keys
-      const uint4* vb = vbuf[b];
+      if (!__all(kp > qmax)) {  // (all: no row of the wave sees a key of the tile)
+        scores(kbuf[b], sc);
+        mask(kp, sc);
+        uint4 pf[RB][2];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const uint4 pf = make_uint4(pack_pair<BF16>(p[2 * h][0], p[2 * h][1]), pack_pair<BF16>(p[2 * h][2], p[2 * h][3]),
-                                    pack_pair<BF16>(p[2 * h + 1][0], p[2 * h + 1][1]),
-                                    pack_pair<BF16>(p[2 * h + 1][2], p[2 * h + 1][3]));
+        for (int rb = 0; rb < RB; ++rb) {
+          new_max(rb, tile_max(sc[rb]));
+          const float mref = m[rb] == -INFINITY ? 0.f : m[rb];
+          float rs = 0.f;
 #pragma unroll
-        for (int j = 0; j < OJ; ++j) {
-          const int vr = 16 * j + (lane & 15);
-          o[j] = mfma16x32<BF16>(vb[vr * 8 + ((4 * h + (lane >> 4)) ^ ((vr >> 1) & 7))], pf, o[j]);
+          for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              sc[rb][c][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[rb][c][i], sl2, -mref));
+              rs += sc[rb][c][i];
+            }
+          l[rb] += rs;  // this lane's keys; the lanes of a row meet at the end
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            pf[rb][h] = make_uint4(pack_pair<BF16>(sc[rb][2 * h][0], sc[rb][2 * h][1]),
+                                   pack_pair<BF16>(sc[rb][2 * h][2], sc[rb][2 * h][3]),
+                                   pack_pair<BF16>(sc[rb][2 * h + 1][0], sc[rb][2 * h + 1][1]),
+                                   pack_pair<BF16>(sc[rb][2 * h + 1][2], sc[rb][2 * h + 1][3]));
         }
-      }
-      wait_vmem();
-      __syncthreads();  // tile t+1 is in LDS everywhere; every wave is done with tile t
+        // O^T += V^T P^T over the two groups of 32 keys
+        const uint4* vb = vbuf[b];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) kp[c] = kpn[c];
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int j = 0; j < OJ; ++j) {
+            const int vr = 16 * j + (lane & 15);
+            const uint4 vf = vb[vr * 8 + ((4 * h + (lane >> 4)) ^ ((vr >> 1) & 7))];
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) o[rb][j] = mfma16x32<BF16>(vf, pf[rb][h], o[rb][j]);
+          }
+      }
+      arrive(kpn);  // tile t + 1 is in LDS everywhere; every wave is done with tile t
+      kp = kpn;
     }
   }
 
-  const int64_t r = row0 + (lane & 15);
-  if (r < rows) {
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    const int64_t r = row0 + 16 * rb + (lane & 15);
+    const float ls = lanes4_sum(l[rb]);
+    if (r >= rows) continue;
     const int d0 = 4 * (lane >> 4);
     if (gridDim.z == 1) {
       const int64_t t = r / a.group, hh = g * a.group + (r - t * a.group);
-      const float inv = 1.0f / fmaxf(l, 1e-12f);
+      const float inv = 1.0f / fmaxf(ls, 1e-12f);
       uint16_t* orow = static_cast<uint16_t*>(a.out) + t * a.out_st + hh * D;
 #pragma unroll
       for (int j = 0; j < OJ; ++j)
         *reinterpret_cast<uint2*>(orow + 16 * j + d0) =
-            make_uint2(pack_pair<BF16>(o[j][0] * inv, o[j][1] * inv), pack_pair<BF16>(o[j][2] * inv, o[j][3] * inv));
+            make_uint2(pack_pair<BF16>(o[rb][j][0] * inv, o[rb][j][1] * inv),
+                       pack_pair<BF16>(o[rb][j][2] * inv, o[rb][j][3] * inv));
     } else {
       float* pr = a.part + ((static_cast<int64_t>(blockIdx.z) * a.hkv + g) * rows + r) * (D + 2);
       if (lane < 16) {
-        pr[0] = m;
-        pr[1] = l;
+        pr[0] = m[rb];
+        pr[1] = ls;
       }
 #pragma unroll
       for (int j = 0; j < OJ; ++j)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) pr[2 + 16 * j + d0 + i] = o[j][i];
+        for (int i = 0; i < 4; ++i) pr[2 + 16 * j + d0 + i] = o[rb][j][i];
     }
   }
 }
@@ -1498,6 +1576,7 @@ static bool flat_form(int64_t rows, int64_t num_entries) {
 
 struct FlatPlan {
   int64_t npad, tiles, splits, tiles_per_split;
+  int rb;  // 16-row blocks per wave
   int64_t part_bytes, kf_bytes, vt_bytes, kp_bytes;
   int64_t total() const { return part_bytes + kf_bytes + vt_bytes + kp_bytes; }
 };
@@ -1513,10 +1592,18 @@ static FlatPlan flat_plan(int64_t rows, int64_t hkv, int64_t num_entries, int64_
   // 256 queries run best at 8 splits (43 us against 51 at 4 and 52 at 16),
   // 1024 queries at 4 (98 against 126 unsplit).  Override
   // BFA_TUNE_CASCADE_FLAT_WG sets the workgroup target instead.
+  // Two 16-row blocks per wave from more than 256 rows (head_dim 64: 1024), where
+  // enough workgroups remain: Llama-3-8B, 100 queries (400 rows) over 8000 keys
+  // 58 -> 53 us, TinyLlama, 1000 (8000 rows) over 3000 71 -> 66 us, but 100 (800
+  // rows) 25 -> 28 us.
+  fp.rb = rows > (d == 64 ? 1024 : 256) ? 2 : 1;
   const int64_t blocks = cdiv(rows, 64) * hkv;
   int64_t target = std::min<int64_t>(std::max<int64_t>(512, 4 * blocks), 1024);
   if (tuning(BFA_TUNE_CASCADE_FLAT_WG) >= 1) target = tuning(BFA_TUNE_CASCADE_FLAT_WG);
-  int64_t zs = std::min<int64_t>(cdiv(target, blocks), fp.tiles);
+  // at least three tiles per split: below that a split's own fill and its share
+  // of the merge cost more than it saves (TinyLlama, 24 queries over 2000 keys:
+  // 17.1 us at one tile per split, 14.6 at three)
+  int64_t zs = std::min<int64_t>(cdiv(target, blocks), cdiv(fp.tiles, 3));
   zs = std::max<int64_t>(1, zs);
   fp.tiles_per_split = std::max<int64_t>(1, cdiv(fp.tiles, zs));
   fp.splits = std::max<int64_t>(1, cdiv(fp.tiles, fp.tiles_per_split));
@@ -1700,13 +1787,14 @@ extern "C" int bfa_cascade_attention(
     f.tiles_per_split = fp.tiles_per_split;
     const hipStream_t s = as_stream(stream);
     const dim3 pgrid(static_cast<unsigned>(fp.tiles), static_cast<unsigned>(num_kv_heads), 2);
-    const dim3 grid(static_cast<unsigned>(cdiv(rows, 64)), static_cast<unsigned>(num_kv_heads),
+    const dim3 grid(static_cast<unsigned>(cdiv(rows, 64 * fp.rb)), static_cast<unsigned>(num_kv_heads),
                     static_cast<unsigned>(fp.splits));
     auto launch = [&](auto bf, auto dd) {
       constexpr bool B = decltype(bf)::value;
       constexpr int DD = decltype(dd)::value;
       hipLaunchKernelGGL((cascade_flatten_kernel<B, DD>), pgrid, dim3(256), 0, s, a, f);
-      hipLaunchKernelGGL((cascade_flat_kernel<B, DD>), grid, dim3(256), 0, s, a, f);
+      if (fp.rb == 2) hipLaunchKernelGGL((cascade_flat_kernel<B, DD, 2>), grid, dim3(256), 0, s, a, f);
+      else hipLaunchKernelGGL((cascade_flat_kernel<B, DD, 1>), grid, dim3(256), 0, s, a, f);
       if (fp.splits > 1) launch_merge<B, DD>(a, rows, fp.splits, s);
     };
     dispatch_dtype_hd(dtype, head_dim, launch);

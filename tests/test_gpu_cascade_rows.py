@@ -1,0 +1,60 @@
+"""The flat form of cascade attention at the edges of its row blocks: one and two
+16-row blocks per wave (from 257 rows per kv head at head_dim 128, 1025 at 64),
+against the oracle; and what its softmax does with scores that keep growing
+along the keys and with a negative scale, against 64 bits."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from braidinfer_amd.layers import CascadeAttention, RotaryEmbedding
+from tests.helpers import assert_close, gen, randn
+from tests.test_gpu_cascade import _check_case, build_case
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("tokens,hq,hkv,d", [(128, 16, 8, 128), (129, 16, 8, 128), (161, 4, 1, 128),
+                                             (128, 32, 4, 64), (129, 32, 4, 64), (145, 16, 2, 64)])
+@pytest.mark.parametrize("causal,knorm", [(True, False), (False, True)])
+def test_row_blocks(tuning, tokens, hq, hkv, d, causal, knorm):
+    tuning("CASCADE_FLAT", 1)
+    _check_case(f"rows {tokens} {hq} {hkv} {d}", tokens, hq, hkv, [48, 130, 64, tokens], [0, 77, -5, 0], causal,
+                knorm, d=d)
+
+
+@pytest.mark.parametrize("tokens", [100, 300])
+@pytest.mark.parametrize("wg", [8, 64])
+def test_growing_scores_and_sign(tuning, tokens, wg):
+    """Keys that grow along the walk move the running maximum in every tile (by
+    less and by more than the step that rescales); P is rounded to bf16 as
+    everywhere, so the plain tolerance holds.  (-q, -scale) is (q, scale)."""
+    tuning("CASCADE_FLAT", 1)
+    tuning("CASCADE_FLAT_WG", wg)
+    hq, hkv, d, ps = 8, 4, 128, 16
+    chunks, kv, total = build_case(91, hq, hkv, [400, 300, 200], [0, 0, 0], pages=90)
+    for i, c in enumerate(chunks):
+        c.cached_position_start -= 1000
+        c.global_position_start -= 1000
+        for j, p in enumerate(c.page_table):
+            kv[p, 0] *= 0.05 + 0.1 * (i + j / 20.0)
+    rope = RotaryEmbedding(d, d, 4096, 1e6).to(DEV)
+    q = randn(gen(92), tokens, hq, d, std=3.0)
+    qpos = torch.arange(total - tokens, total)
+    outs = []
+    for s in (1.0, -1.0):
+        att = CascadeAttention(hq, d, s * d ** -0.5, hkv, ps, rotary_emb=rope)
+        levels = att.create_cascade_levels(chunks)
+        outs.append(att.forward((q * s).to(DEV), qpos.to(DEV), kv.to(DEV), levels, 0).cpu())
+    assert torch.equal(outs[0], outs[1])
+    ks, vs = [], []
+    for c in chunks:
+        k, v = (kv[c.page_table, i].double().transpose(1, 2).reshape(-1, hkv, d)[: c.kv_length] for i in (0, 1))
+        ks.append(k)
+        vs.append(v)
+    k, v = torch.cat(ks).repeat_interleave(hq // hkv, 1), torch.cat(vs).repeat_interleave(hq // hkv, 1)
+    sc = torch.einsum("thd,khd->htk", q.double(), k) * d ** -0.5
+    hide = torch.arange(total)[None, :] > qpos[:, None]
+    exp = torch.einsum("htk,khd->thd", torch.softmax(sc.masked_fill(hide, float("-inf")), -1), v)
+    assert_close(outs[0].reshape(tokens, hq, d), exp, what=f"growing scores tokens={tokens} wg={wg}")
