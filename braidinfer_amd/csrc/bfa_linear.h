@@ -1,5 +1,6 @@
-// The linear-layer GEMM for 65 and more tokens (linear_gemm.hip), launched by
-// bfa_linear (qkv.hip).
+// The linear-layer kernels that bfa_linear (qkv.hip) launches: the GEMM for 65 and
+// more tokens (linear_gemm.hip) and the one-launch weight stream for few
+// (linear_gemv.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -33,5 +34,9 @@ struct LinArgs {
 // split = false: without split K, so without a workspace.
 GemmPlan linear_plan(int64_t m, int64_t n, int64_t k, bool swiglu, bool split);
 void launch_linear_gemm(const GemmPlan& p, LinArgs q, int dt, hipStream_t st);
+
+// One launch, no workspace (of LinArgs: part and the planner's fields unused).
+bool linear_gemv_ok(int64_t m, int64_t wrows, int64_t k);
+void launch_linear_gemv(LinArgs q, int dt, hipStream_t st);
 
 }  // namespace bfa

@@ -3306,6 +3306,7 @@ extern "C" int bfa_fused_rmsnorm_qkv_noalloc(
 extern "C" int64_t bfa_linear_workspace_size(int64_t tokens, int64_t k, int64_t n, int mode) {
   if (tokens <= 0 || n <= 0) return 0;
   const int64_t nw = mode == BFA_LINEAR_SILU_AND_MUL ? 2 * n : n;
+  if (linear_gemv_ok(tokens, nw, k)) return 0;
   const QkvPlan p = make_plan(tokens, nw, k, 0);
   if (p.decode) return p.part_bytes;
   // above 64 tokens: the fp32 partials of the tiles that are split over K; a
@@ -3338,6 +3339,31 @@ extern "C" int bfa_linear(const void* x, int dtype, int64_t tokens, int64_t k, i
   BFA_REQUIRE(x && weight && out, "%s: null pointer", what);
   const bool swiglu = mode == BFA_LINEAR_SILU_AND_MUL;
   const int64_t nw = swiglu ? 2 * n : n;
+  const hipStream_t st = as_stream(stream);
+  const bool vec = aligned16(out) && out_stride % 8 == 0 &&
+                   (residual == nullptr || (aligned16(residual) && residual_stride % 8 == 0));
+  const bool gemv = linear_gemv_ok(tokens, nw, k);
+  if (gemv || (tokens > 64 && k % 64 == 0 && tokens * x_stride * 2 < (int64_t(1) << 32) &&
+               nw * w_stride * 2 < (int64_t(1) << 32))) {
+    LinArgs q{};
+    q.a = static_cast<const uint16_t*>(x);
+    q.w = static_cast<const uint16_t*>(weight);
+    q.m = tokens; q.n = n; q.k = k; q.lda = x_stride; q.ldw = w_stride;
+    q.bias = bias; q.bias_dt = bias_dtype; q.res = residual; q.res_dt = residual_dtype; q.ldr = residual_stride;
+    q.out = out; q.ldo = out_stride;
+    q.proj_dt = proj_dtype; q.mid_dt = sum_dtype; q.out_dt = out_dtype;
+    q.vec = vec; q.swiglu = swiglu ? 1 : 0;
+    if (gemv) {
+      launch_linear_gemv(q, dtype, st);
+      return check_launch(what);
+    }
+    GemmPlan lp = linear_plan(tokens, n, k, swiglu, true);
+    if (lp.part_bytes > 0 && (workspace_bytes < lp.part_bytes || !workspace || !aligned16(workspace)))
+      lp = linear_plan(tokens, n, k, swiglu, false);
+    q.part = static_cast<float*>(workspace);
+    launch_linear_gemm(lp, q, dtype, st);
+    return check_launch(what);
+  }
   const QkvPlan p = make_plan(tokens, nw, k, 0);
   const int64_t need = p.decode ? p.part_bytes : 0;
   BFA_REQUIRE(workspace_bytes >= need && (need == 0 || workspace),
@@ -3350,13 +3376,11 @@ extern "C" int bfa_linear(const void* x, int dtype, int64_t tokens, int64_t k, i
   e.res = residual; e.res_dt = residual_dtype; e.ldr = residual_stride;
   e.bias = bias; e.bias_dtype = bias_dtype;
   e.out = out; e.ldo = out_stride; e.n = n;
-  e.vec = aligned16(out) && out_stride % 8 == 0 &&
-          (residual == nullptr || (aligned16(residual) && residual_stride % 8 == 0));
+  e.vec = vec;
   GemmArgs g{};
   g.a = static_cast<const uint16_t*>(x);
   g.w = static_cast<const uint16_t*>(weight);
   g.m = tokens; g.n = n; g.k = k; g.lda = x_stride; g.ldw = w_stride;
-  const hipStream_t st = as_stream(stream);
   const bool bf16 = dtype == BFA_DTYPE_BF16;
   if (p.decode) {
     SplitArgs sa{};
@@ -3377,20 +3401,6 @@ extern "C" int bfa_linear(const void* x, int dtype, int64_t tokens, int64_t k, i
       hipLaunchKernelGGL(linear_decode_epilogue_kernel<false>, egrid, dim3(256), 0, st, part, p.splits,
                          reg_order, p.mt, tokens, nw, g, e);
     }
-    return check_launch(what);
-  }
-  if (k % 64 == 0 && tokens * x_stride * 2 < (int64_t(1) << 32) && nw * w_stride * 2 < (int64_t(1) << 32)) {
-    LinArgs q{};
-    q.a = g.a; q.w = g.w; q.m = tokens; q.n = n; q.k = k; q.lda = x_stride; q.ldw = w_stride;
-    q.bias = bias; q.bias_dt = bias_dtype; q.res = residual; q.res_dt = residual_dtype; q.ldr = residual_stride;
-    q.out = out; q.ldo = out_stride;
-    q.proj_dt = proj_dtype; q.mid_dt = sum_dtype; q.out_dt = out_dtype;
-    q.vec = e.vec; q.swiglu = swiglu ? 1 : 0;
-    GemmPlan lp = linear_plan(tokens, n, k, swiglu, true);
-    if (lp.part_bytes > 0 && (workspace_bytes < lp.part_bytes || !workspace || !aligned16(workspace)))
-      lp = linear_plan(tokens, n, k, swiglu, false);
-    q.part = static_cast<float*>(workspace);
-    launch_linear_gemm(lp, q, dtype, st);
     return check_launch(what);
   }
   if (bf16) launch_linear<true>(g, e, swiglu, st); else launch_linear<false>(g, e, swiglu, st);

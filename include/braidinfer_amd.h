@@ -80,7 +80,9 @@ const char* bfa_last_error(void);
                                         (1-8 tokens without q/k norm) */
 #define BFA_TUNE_GEMM_TILE 13      /* BFA_GEMM_TILE: tile id of the GEMMs above 64 tokens (0-7) */
 #define BFA_TUNE_GEMM_SPLITS 14    /* BFA_GEMM_SPLITS: its K splits */
-#define BFA_TUNE_COUNT 15
+#define BFA_TUNE_LINEAR_GEMV 15      /* BFA_LINEAR_GEMV: 0 = never the one-launch linear kernel,
+                                      non-zero = for every call of up to 64 tokens */
+#define BFA_TUNE_COUNT 16
 int bfa_set_tuning(int key, int value);
 int bfa_get_tuning(int key);
 
