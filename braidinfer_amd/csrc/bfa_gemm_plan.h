@@ -62,10 +62,11 @@ struct GemmPlan {
 // Each tile is weighed with every tile whole and, where the last round is not
 // full, with that round's tiles split over K as often as the CUs allow: rounds
 // times (stages x stage_us + fixed_us for fill and epilogue), and for split
-// tiles the second launch (4 us) and the partials' round trip (3 TB/s), which
+// tiles the second launch (split_us) and the partials' round trip (3 TB/s), which
 // may take up to part_limit bytes.  Overrides: BFA_TUNE_GEMM_TILE,
 // BFA_TUNE_GEMM_SPLITS.
-inline GemmPlan gemm_plan(int64_t m, int64_t wrows, int64_t k, double fixed_us, int64_t part_limit) {
+inline GemmPlan gemm_plan(int64_t m, int64_t wrows, int64_t k, double fixed_us, double split_us,
+                          int64_t part_limit) {
   const int ot = tuning(BFA_TUNE_GEMM_TILE), os = tuning(BFA_TUNE_GEMM_SPLITS);
   const int64_t kt = k / 64;
   GemmPlan best{};
@@ -88,7 +89,7 @@ inline GemmPlan gemm_plan(int64_t m, int64_t wrows, int64_t k, double fixed_us, 
     const int64_t bytes = rest * s * t.rw * t.cw * t.ma * 4 * 64 * 16;
     if (rest > 0 && s > 1 && bytes <= part_limit) {
       const double cs = static_cast<double>(rounds) * (kt * t.stage_us + fixed_us) +
-                        static_cast<double>(cdiv(rest * s, 256)) * (cdiv(kt, s) * t.stage_us + fixed_us) + 4.0 +
+                        static_cast<double>(cdiv(rest * s, 256)) * (cdiv(kt, s) * t.stage_us + fixed_us) + split_us +
                         static_cast<double>(bytes) / 3.0e6;
       if (cs < c || os > 1) {
         c = cs;

@@ -32,8 +32,4 @@ int fill_append_args(const char* what, void* layer_cache, int cache_dtype, int64
                      const void* positions, int positions_dtype, int64_t page_size, int32_t* status,
                      AppendArgs* out);
 
-// slot_off[t] = element offset of token t's cache slot (page * stride_page +
-// slot * stride_slot), or -1 when the append rule skips it (status flagged).
-void launch_kv_slots(const AppendArgs& a, int64_t tokens, int64_t* slot_off, hipStream_t s);
-
 }  // namespace bfa

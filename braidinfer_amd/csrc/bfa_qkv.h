@@ -47,19 +47,15 @@ struct QkvEpi {
   int64_t hidden;
   float stat_eps;
   // Paged-KV append in the epilogue (bfa_fused_rmsnorm_qkv_append): the k and v
-  // heads of row t also go to cache + slot_off[t] + (V ? c_skv : 0) + (head -
+  // heads of row t also go to cache + slot(t) + (V ? c_skv : 0) + (head -
   // first head of its kind) * c_sh + column in the head, as cache_dt (from the
-  // value rounded to out_dt); slot_off[t] < 0 skips the row.  skip_kv_out = 1
+  // value rounded to out_dt); a token without a slot is skipped.  skip_kv_out = 1
   // leaves the k/v columns of `out` unwritten.
   void* cache;
   int cache_dt;
   int64_t c_skv, c_sh;
-  const int64_t* slot_off;
   int skip_kv_out;
-  // app_in_kernel = 1: the prefill GEMM resolves its rows' cache slots itself
-  // (before the K loop, from `app`), and slot_off is not used
-  int app_in_kernel;
-  AppendArgs app;
+  AppendArgs app;  // how a token's slot is found: by the epilogues themselves
   // prefill with the norm weight folded into W (the fp32 variants): the
   // projection of row t is multiplied by row_scale[t] (1 / rms) before the bias
   const float* row_scale;
@@ -204,7 +200,6 @@ struct GemvKArgs {
   void* out;
   int* status;
   void* cache;
-  const int64_t* slot_off;
   int64_t ldo, c_skv, c_sh;
   int32_t m, k, lda, ldw, pw, hq, hkv, hd, max_pos;
   float eps;

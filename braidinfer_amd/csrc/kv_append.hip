@@ -129,23 +129,6 @@ __global__ __launch_bounds__(256) void kv_append_scalar_kernel(AppendArgs a) {
   }
 }
 
-// Cache slot of every token for the QKV epilogues that append K and V
-// themselves: slot_off[t] = page * c_sp + slot * c_ss (elements), or -1 when the
-// token is not written (the reason is flagged in the status word).
-__global__ __launch_bounds__(256) void kv_slot_kernel(AppendArgs a, int64_t tokens, int64_t* slot_off) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (t >= tokens) return;
-  int64_t page = 0, slot = 0;
-  const int bad = append_target_code(a, t, page, slot);
-  if (bad) flag_status(a.status, bad);
-  slot_off[t] = bad ? -1 : page * a.c_sp + slot * a.c_ss;
-}
-
-void launch_kv_slots(const AppendArgs& a, int64_t tokens, int64_t* slot_off, hipStream_t s) {
-  hipLaunchKernelGGL(kv_slot_kernel, dim3(static_cast<unsigned>(cdiv(tokens, 256))), dim3(256), 0, s, a,
-                     tokens, slot_off);
-}
-
 int fill_append_args(const char* what, void* layer_cache, int cache_dtype, int64_t num_pages,
                      int64_t cache_page_slots, int64_t stride_page, int64_t stride_kv,
                      int64_t stride_head, int64_t stride_slot, const void* kv_indices,

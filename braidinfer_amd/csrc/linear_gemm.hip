@@ -214,7 +214,7 @@ void launch_form(const GemmPlan& p, const LinArgs& q, hipStream_t st) {
 }  // namespace
 
 GemmPlan linear_plan(int64_t m, int64_t n, int64_t k, bool swiglu, bool split) {
-  return gemm_plan(m, swiglu ? 2 * n : n, k, 4.0, split ? INT64_MAX : 0);
+  return gemm_plan(m, swiglu ? 2 * n : n, k, 4.0, 4.0, split ? INT64_MAX : 0);
 }
 
 void launch_linear_gemm(const GemmPlan& p, LinArgs q, int dt, hipStream_t st) {

@@ -586,11 +586,6 @@ __device__ __forceinline__ void gemm_epilogue(ACC& acc, uint4* lds, const GemmAr
       }
     }
     __syncthreads();
-    if (e.cache != nullptr && !e.app_in_kernel) {
-      // rows past m read the last row's slot; their stores are masked
-      for (int r = lane; r < MB * 32; r += 64) stab[r] = e.slot_off[min(wrow0 + r, g.m - 1)];
-      __asm__ volatile("" ::: "memory");  // the wave's own LDS writes precede its reads below
-    }
     // Row scales (the norm weight folded into W): this wave's rows go to a
     // wave-private LDS table after the slot tables, read once per row below
     // (held in registers a block ahead, they had made the epilogue spill).
@@ -787,14 +782,10 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, (WM * WN <= 8192 ? 2 : 
   // page-table lookups wait together with those loads, not ahead of them.
   auto resolve_slots = [&]() {
     if constexpr (EPI == EPI_FUSED) {
-      if (e.cache != nullptr && e.app_in_kernel) {
+      if (e.cache != nullptr) {
         int64_t* stab = reinterpret_cast<int64_t*>(lds + SLOT_U4) + wid * (MB * 32);
-        for (int r = lane; r < MB * 32; r += 64) {
-          int64_t page = 0, slot = 0;
-          const int bad = append_target_code(e.app, min(m0 + wm * WM + r, g.m - 1), page, slot);
-          if (bad) flag_status(e.app.status, bad);
-          stab[r] = bad ? -1 : page * e.app.c_sp + slot * e.app.c_ss;
-        }
+        for (int r = lane; r < MB * 32; r += 64)
+          stab[r] = append_slot(e.app, append_key(e.app, min(m0 + wm * WM + r, g.m - 1)));
       }
     }
   };
@@ -1556,7 +1547,7 @@ __global__ __launch_bounds__(256) void qkv_decode_loop_kernel(DecodeArgs d, int 
 // consecutive bytes.  The splits are summed in order (deterministic), then each
 // token goes through bias -> rounding -> per-head RMSNorm (a wave reduction per
 // token) -> rounding -> RoPE -> store, as in the prefill epilogue.
-template <int MAXP>  // RoPE pairs per lane: head_dim <= 2 * 64 * MAXP
+template <int MAXP, bool APP>  // APP: the call appends k and v (its code costs the plain call 1 us of 18)
 __device__ __forceinline__ void decode_epilogue_item(const float4* part, int64_t splits,
                                                               int64_t ntiles, int mt, int64_t m,
                                                               const QkvEpi& e, int64_t tg, int64_t h,
@@ -1578,13 +1569,11 @@ __device__ __forceinline__ void decode_epilogue_item(const float4* part, int64_t
   // values masked) so that none waits behind a per-token or per-dtype branch.
   // absent inputs read a valid stand-in (the partials) and are masked after
   const void* posp = rope ? e.positions : part;
-  // fused KV append: cache slots of the 4 tokens (first load level)
-  const bool app = e.cache != nullptr && kd != 0;
-  int64_t so[4] = {-1, -1, -1, -1};
-  if (app) {
-#pragma unroll
-    for (int v = 0; v < 4; ++v) so[v] = e.slot_off[min(tg * 4 + v, m - 1)];
-  }
+  // fused KV append: lane l finds the slot of token l % 4 (its key in the first
+  // load level)
+  const bool app = APP && kd != 0;
+  AppendKey akey{0, 0};
+  if (app) akey = append_key(e.app, min(tg * 4 + (lane & 3), m - 1));
   int64_t raw[4];
   if (rope && e.pos_is_i64) {
 #pragma unroll
@@ -1650,6 +1639,9 @@ __device__ __forceinline__ void decode_epilogue_item(const float4* part, int64_t
     if (e.bias) load2_any(e.bias, e.bias_dtype, base + pc, base + half + pc, b1[pp], b2[pp]);
     if (nw) load2_any(nw, e.qk_w_dtype, pc, half + pc, g1[pp], g2[pp]);
   }
+  // the page table's loads, behind the others in flight
+  int64_t my_so = -1;
+  if (app) my_so = append_slot(e.app, akey);
   asm volatile("" ::: "memory");
   float4 a1[MAXP], a2[MAXP];
 #pragma unroll
@@ -1746,6 +1738,12 @@ __device__ __forceinline__ void decode_epilogue_item(const float4* part, int64_t
   for (int v = 0; v < 4; ++v) {
     const int64_t t = tg * 4 + v;
     if (t >= m) continue;
+    int64_t so = -1;
+    if (app) {  // lane v holds token v's slot
+      const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(my_so), v));
+      const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(my_so >> 32), v));
+      so = static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
+    }
 #pragma unroll
     for (int pp = 0; pp < MAXP; ++pp) {
       const int64_t p = lane + 64 * pp;
@@ -1760,9 +1758,9 @@ __device__ __forceinline__ void decode_epilogue_item(const float4* part, int64_t
         store_any(e.out, e.out_dt, t * e.ldo + base + p, a);
         store_any(e.out, e.out_dt, t * e.ldo + base + half + p, b);
       }
-      if (app && so[v] >= 0) {
+      if (so >= 0) {
         const int64_t hk = h - e.hq - (kd == 2 ? e.hkv : 0);
-        const int64_t cb = so[v] + (kd == 2 ? e.c_skv : 0) + hk * e.c_sh;
+        const int64_t cb = so + (kd == 2 ? e.c_skv : 0) + hk * e.c_sh;
         store_any(e.cache, e.cache_dt, cb + p, round_to(a, e.out_dt));
         store_any(e.cache, e.cache_dt, cb + half + p, round_to(b, e.out_dt));
       }
@@ -1859,7 +1857,7 @@ __global__ __launch_bounds__(256) void linear_decode_epilogue_kernel(const float
   }
 }
 
-template <int MAXP>
+template <int MAXP, bool APP>
 __global__ __launch_bounds__(256) void qkv_decode_epilogue_kernel(const float4* part, int64_t splits,
                                                                   int64_t ntiles, int mt, int64_t m,
                                                                   QkvEpi e) {
@@ -1867,7 +1865,7 @@ __global__ __launch_bounds__(256) void qkv_decode_epilogue_kernel(const float4* 
   const int64_t item = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (item >= cdiv(m, 4) * heads) return;
   const int64_t tg = item / heads;
-  decode_epilogue_item<MAXP>(part, splits, ntiles, mt, m, e, tg, item - tg * heads, threadIdx.x & 63);
+  decode_epilogue_item<MAXP, APP>(part, splits, ntiles, mt, m, e, tg, item - tg * heads, threadIdx.x & 63);
 }
 
 // ================================== decode: whole-K column-pair tiles
@@ -2030,7 +2028,7 @@ __global__ __launch_bounds__(256) void qkv_decode_pair_kernel(DecodeArgs d, QkvE
   }
   float cs[4] = {1.f, 1.f, 1.f, 1.f}, sn[4] = {0.f, 0.f, 0.f, 0.f};
   uint32_t bw[4] = {0, 0, 0, 0};
-  int64_t so[4] = {-1, -1, -1, -1};
+  AppendKey akey{0, 0};  // of token 16 wid + lane % 16
   bool pok[4] = {true, true, true, true};
   const bool app = e.cache != nullptr && kd != 0;
   const int64_t p = c0 + lr;  // this lane's pair inside the head
@@ -2042,10 +2040,7 @@ __global__ __launch_bounds__(256) void qkv_decode_pair_kernel(DecodeArgs d, QkvE
       const int64_t ia = (cola + lr) << sh, ib = (cola + half + lr) << sh;
       bw[0] = bp[ia]; bw[1] = bp[ia + sh]; bw[2] = bp[ib]; bw[3] = bp[ib + sh];
     }
-    if (app) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) so[v] = e.slot_off[min<int64_t>(wid * 16 + lq * 4 + v, d.m - 1)];
-    }
+    if (app) akey = append_key(e.app, min<int64_t>(wid * 16 + lr, d.m - 1));
   }
   auto rope_loads = [&]() {
     if (wid >= MT || !rope) return;
@@ -2159,6 +2154,10 @@ __global__ __launch_bounds__(256) void qkv_decode_pair_kernel(DecodeArgs d, QkvE
     }
   }
 
+  // the cache slots: the page table's loads fly while the partial tiles meet
+  int64_t my_so = -1;
+  if (app && wid < MT) my_so = append_slot(e.app, akey);
+
   // the four partial tiles (and Gram diagonals) through each wave's own ring
   float4* mine = reinterpret_cast<float4*>(ring + wid * WAVE_U4);
 #pragma unroll
@@ -2215,6 +2214,9 @@ __global__ __launch_bounds__(256) void qkv_decode_pair_kernel(DecodeArgs d, QkvE
     }
   }
   const int64_t hk = head - e.hq - (kd == 2 ? e.hkv : 0);
+  int64_t so[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) so[v] = __shfl(my_so, lq * 4 + v);
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
     const int64_t t = i * 16 + lq * 4 + v;
@@ -2266,7 +2268,6 @@ __device__ __forceinline__ void row_epilogue_item(const float* part, int64_t spl
   const int32_t* p32 = static_cast<const int32_t*>(rope ? e.positions : static_cast<const void*>(pr));
   const int32_t plo = p32[!rope ? 0 : (e.pos_is_i64 ? 2 * t : t)];
   const int32_t phi = p32[!rope ? 0 : (e.pos_is_i64 ? 2 * t + 1 : t)];
-  const int64_t so_raw = (app ? e.slot_off : reinterpret_cast<const int64_t*>(part))[app ? t : 0];
   int64_t jj[MAXP];
   bool jin[MAXP];
   uint32_t bw1[MAXP], bw2[MAXP], nw1[MAXP], nw2[MAXP];
@@ -2310,6 +2311,8 @@ __device__ __forceinline__ void row_epilogue_item(const float* part, int64_t spl
     cv[p] = csr[rope ? jj[p] : 0];
     sv[p] = csr[rope ? half + jj[p] : 0];
   }
+  // the cache slot, while the loads above are on their way
+  const int64_t so = app ? append_slot(e.app, append_key(e.app, t)) : -1;
   // the split sums, in split order
   for (int64_t sp0 = 0;;) {
 #pragma unroll
@@ -2357,7 +2360,6 @@ __device__ __forceinline__ void row_epilogue_item(const float* part, int64_t spl
       x2[p] = ok ? round_to(b * cv[p] + a * sv[p], dt) : 0.f;
     }
   }
-  const int64_t so = app ? so_raw : -1;
   const int64_t cb = so + (kd == 2 ? e.c_skv : 0) + (h - e.hq - (kd == 2 ? e.hkv : 0)) * e.c_sh;
 #pragma unroll
   for (int p = 0; p < MAXP; ++p) {
@@ -2783,9 +2785,8 @@ struct CacheEpi {
   void* cache;
   int cache_dt;
   int64_t c_skv, c_sh;
-  const int64_t* slot_off;  // resolved slots (decode and raw-epilogue paths)
   int skip_kv_out;
-  const AppendArgs* app;    // the prefill GEMM's fused epilogue resolves its own
+  const AppendArgs* app;
 };
 
 // The projection with its epilogue; `operand` rows are `lda` apart.  With a
@@ -2853,13 +2854,8 @@ static int qkv_projection_impl(const void* operand, int64_t lda, const OperandFo
   }
   if (ce) {
     e.cache = ce->cache; e.cache_dt = ce->cache_dt; e.c_skv = ce->c_skv; e.c_sh = ce->c_sh;
-    e.slot_off = ce->slot_off; e.skip_kv_out = ce->skip_kv_out;
-    if (!p.decode && p.fused_epi) {
-      e.app_in_kernel = 1;
-      e.app = *ce->app;
-    } else {
-      BFA_REQUIRE(ce->slot_off != nullptr, "%s: cache slots not resolved", what);
-    }
+    e.skip_kv_out = ce->skip_kv_out;
+    e.app = *ce->app;
   }
 
   const hipStream_t st = as_stream(stream);
@@ -2914,16 +2910,19 @@ static int qkv_projection_impl(const void* operand, int64_t lda, const OperandFo
       const int64_t items = cdiv(tokens, 4) * heads;
       const dim3 grid(static_cast<unsigned>(cdiv(items, 4)));
       const float4* p4 = reinterpret_cast<const float4*>(part);
-      if (hd <= 128) {
-        hipLaunchKernelGGL(qkv_decode_epilogue_kernel<1>, grid, dim3(256), 0, st, p4, p.splits,
-                           cdiv(qkv_dim, 128), p.mt, tokens, e);
-      } else if (hd <= 256) {
-        hipLaunchKernelGGL(qkv_decode_epilogue_kernel<2>, grid, dim3(256), 0, st, p4, p.splits,
-                           cdiv(qkv_dim, 128), p.mt, tokens, e);
-      } else {
-        hipLaunchKernelGGL(qkv_decode_epilogue_kernel<4>, grid, dim3(256), 0, st, p4, p.splits,
-                           cdiv(qkv_dim, 128), p.mt, tokens, e);
-      }
+      auto launch = [&](auto maxp) {
+        constexpr int P = decltype(maxp)::value;
+        if (e.cache) {
+          hipLaunchKernelGGL((qkv_decode_epilogue_kernel<P, true>), grid, dim3(256), 0, st, p4, p.splits,
+                             cdiv(qkv_dim, 128), p.mt, tokens, e);
+        } else {
+          hipLaunchKernelGGL((qkv_decode_epilogue_kernel<P, false>), grid, dim3(256), 0, st, p4, p.splits,
+                             cdiv(qkv_dim, 128), p.mt, tokens, e);
+        }
+      };
+      if (hd <= 128) launch(std::integral_constant<int, 1>{});
+      else if (hd <= 256) launch(std::integral_constant<int, 2>{});
+      else launch(std::integral_constant<int, 4>{});
     } else {
       launch_epilogue(part, p.splits, tokens, e, st);
     }
@@ -3067,9 +3066,9 @@ extern "C" int bfa_fused_rmsnorm_qkv(const void* x, int x_dtype, int64_t tokens,
 // ------------------------------------------------ fused QKV + paged KV append
 // bfa_fused_rmsnorm_qkv, then bfa_append_paged_kv of its k and v heads (as
 // [tokens, num_kv_heads, head_dim] views of `out`), in the projection's own
-// epilogue: a small kernel first resolves every token's cache slot into the
-// workspace tail (tokens x 8 bytes), then each epilogue writes the finished k/v
-// head rows to the cache as well (and, with write_kv_out = 0, only there).
+// epilogue: each epilogue finds its tokens' cache slots and writes the finished
+// k/v head rows to the cache as well (and, with write_kv_out = 0, only there).
+// A kernel that resolved the slots first cost 3.5 us of a 64-token decode call.
 extern "C" int64_t bfa_fused_rmsnorm_qkv_append_workspace_size(int64_t tokens, int64_t hidden,
                                                                int64_t qkv_dim, int64_t head_dim) {
   if (tokens <= 0) return 0;
@@ -3122,25 +3121,15 @@ extern "C" int bfa_fused_rmsnorm_qkv_append(
   const int64_t heads = num_q_heads + 2 * num_kv_heads;
   BFA_REQUIRE(heads > 0 && qkv_dim % heads == 0, "%s: bad head geometry", what);
   const QkvPlan p = make_plan(tokens, qkv_dim, hidden, qkv_dim / heads);
-  const int64_t need = p.operand_bytes + p.need_bytes + align256(tokens * 8);
+  const int64_t need = p.operand_bytes + p.need_bytes + align256(tokens * 8);  // (the size this entry has always asked for)
   BFA_REQUIRE(workspace && aligned16(workspace) && workspace_bytes >= need,
               "%s: workspace too small (%lld < %lld bytes)", what, (long long)workspace_bytes, (long long)need);
-  // the prefill GEMM with the fused epilogue resolves the slots itself; every
-  // other path reads them from the workspace tail, filled by a small kernel
-  const int64_t fsize = workspace_bytes - align256(tokens * 8);
-  int64_t* slot_off = nullptr;
-  if (p.decode || !p.fused_epi) {
-    slot_off = reinterpret_cast<int64_t*>(static_cast<char*>(workspace) + p.operand_bytes + p.need_bytes);
-    launch_kv_slots(a, tokens, slot_off, as_stream(stream));
-    rc = check_launch(what);
-    if (rc != BFA_OK) return rc;
-  }
-  const CacheEpi ce{layer_cache, cache_dtype, stride_kv, stride_head, slot_off, write_kv_out ? 0 : 1, &a};
+  const CacheEpi ce{layer_cache, cache_dtype, stride_kv, stride_head, write_kv_out ? 0 : 1, &a};
   return fused_impl(x, x_dtype, tokens, hidden, x_stride, norm_weight, nw_dtype, eps, mixed_rounding,
                     qkv_weight, w_dtype, qkv_dim, w_stride, bias, bias_dtype, num_q_heads, num_kv_heads,
                     qkv_dtype, q_norm_weight, k_norm_weight, qk_norm_dtype, qk_eps, qk_norm_out_dtype,
                     positions, positions_dtype, cos_sin_cache, max_position, out, out_dtype, out_stride,
-                    workspace, fsize, status, stream, &ce);
+                    workspace, workspace_bytes, status, stream, &ce);
 }
 
 // The fp32 variants' prefill with the norm weight folded into the QKV weight
@@ -3186,32 +3175,23 @@ extern "C" int bfa_fused_rmsnorm_qkv_folded(
                      "%s: the prefill epilogue (more than 64 tokens, head_dim 32, 64 or 128) or the "
                      "column-pair decode shapes (17-64 bf16 tokens) only", what);
   const int64_t need = p.operand_bytes + p.need_bytes + (layer_cache && p.decode ? align256(tokens * 8) : 0);
-  const int64_t fsize = p.decode ? p.operand_bytes + p.need_bytes : workspace_bytes;
   BFA_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace),
               "%s: workspace too small (%lld < %lld bytes)", what, (long long)workspace_bytes, (long long)need);
   char* ws = static_cast<char*>(workspace);
   if (pair) {
-    int64_t* slot_off = nullptr;
-    if (layer_cache) {
-      slot_off = reinterpret_cast<int64_t*>(ws + fsize);
-      launch_kv_slots(a, tokens, slot_off, as_stream(stream));
-      const int rc = check_launch(what);
-      if (rc != BFA_OK) return rc;
-    }
-    const CacheEpi ce{layer_cache, cache_dtype, stride_kv, stride_head, slot_off, write_kv_out ? 0 : 1, &a};
+    const CacheEpi ce{layer_cache, cache_dtype, stride_kv, stride_head, write_kv_out ? 0 : 1, &a};
     const OperandFold f{nullptr, BFA_DTYPE_BF16, false, eps, 0, reinterpret_cast<float*>(ws)};
     return qkv_projection_impl(x, x_stride, &f, tokens, hidden, folded_weight, w_dtype, qkv_dim, w_stride, bias,
                                bias_dtype, num_q_heads, num_kv_heads, qkv_dtype, nullptr, nullptr, 0, 0.f,
                                BFA_DTYPE_BF16, positions, positions_dtype, cos_sin_cache, max_position, out,
-                               out_dtype, out_stride, ws + p.operand_bytes, fsize - p.operand_bytes, status,
+                               out_dtype, out_stride, ws + p.operand_bytes, workspace_bytes - p.operand_bytes, status,
                                stream, layer_cache ? &ce : nullptr);
   }
   float* rs = static_cast<float*>(workspace);
   const int64_t rs_bytes = align256(tokens * 4);
   int rc = launch_row_scale(x, x_dtype, tokens, hidden, x_stride, rs, eps, as_stream(stream));
   if (rc != BFA_OK) return rc;
-  // the prefill GEMM's fused epilogue resolves the cache slots itself
-  const CacheEpi ce{layer_cache, cache_dtype, stride_kv, stride_head, nullptr, write_kv_out ? 0 : 1, &a};
+  const CacheEpi ce{layer_cache, cache_dtype, stride_kv, stride_head, write_kv_out ? 0 : 1, &a};
   return qkv_projection_impl(x, x_stride, nullptr, tokens, hidden, folded_weight, w_dtype, qkv_dim, w_stride,
                              bias, bias_dtype, num_q_heads, num_kv_heads, qkv_dtype, nullptr, nullptr, 0, 0.f,
                              BFA_DTYPE_BF16, positions, positions_dtype, cos_sin_cache, max_position, out,

@@ -32,11 +32,11 @@ typedef __attribute__((ext_vector_type(4))) float gemv_f32x4_t;
 // layout (lane l: row l % 16, K offset 8 (l / 16)); the four partial tiles meet
 // in LDS and one thread per (token, pair) runs the epilogue.
 template <int TM, bool FOLD>
-__global__ __launch_bounds__(256) void qkv_gemv_kernel(GemvKArgs c) {
+__global__ __launch_bounds__(256) void qkv_gemv_kernel(GemvKArgs c, AppendArgs aa) {
   // every argument goes into registers here, with one wait for their loads
   // (left to the compiler they come in several dependent rounds)
   asm volatile("" ::"s"(c.a), "s"(c.w), "s"(c.gamma), "s"(c.bias), "s"(c.positions), "s"(c.cs), "s"(c.out),
-               "s"(c.status), "s"(c.cache), "s"(c.slot_off));
+               "s"(c.status), "s"(c.cache));
   asm volatile("" ::"s"(c.ldo), "s"(c.c_skv), "s"(c.c_sh), "s"(c.m), "s"(c.k), "s"(c.lda), "s"(c.ldw), "s"(c.pw),
                "s"(c.hq), "s"(c.hkv), "s"(c.hd), "s"(c.max_pos), "s"(c.eps));
   asm volatile("" ::"s"(static_cast<int>(c.gamma_dt)), "s"(static_cast<int>(c.mixed)), "s"(static_cast<int>(c.bias_dt)),
@@ -106,7 +106,6 @@ __global__ __launch_bounds__(256) void qkv_gemv_kernel(GemvKArgs c) {
   const int bdt = c.bias ? c.bias_dt : BFA_DTYPE_BF16;
   const uint32_t bw1 = ld_word_al4(c.bias ? c.bias : own, bdt, c.bias ? ec1 : 0);
   const uint32_t bw2 = ld_word_al4(c.bias ? c.bias : own, bdt, c.bias ? ec2 : 0);
-  const int64_t so_raw = (app ? c.slot_off : reinterpret_cast<const int64_t*>(own))[app ? et : 0];
   // ---- the first weight batch
   uint4 wb[SB];
 #pragma unroll
@@ -121,7 +120,6 @@ __global__ __launch_bounds__(256) void qkv_gemv_kernel(GemvKArgs c) {
   const float cv = csr[rope ? c0 + ep_p : 0];
   const float sv = csr[rope ? half + c0 + ep_p : 0];
   const float b1 = c.bias ? word_value_al4(bw1, bdt, ec1) : 0.f, b2 = c.bias ? word_value_al4(bw2, bdt, ec2) : 0.f;
-  const int64_t so = app ? so_raw : -1;
 
   // ---- operand rows -> LDS (normalised by the fold: round(x / rms(x) * gamma),
   //      the operand pre-pass's rounding points)
@@ -226,6 +224,8 @@ __global__ __launch_bounds__(256) void qkv_gemv_kernel(GemvKArgs c) {
       for (int i = 0; i < SB; ++i) wb[i] = wn[i];
     }
   }
+  // the cache slot (its arguments are read by the k and v heads of an append only)
+  const int64_t so = app && ep ? append_slot(aa, append_key(aa, et)) : -1;
   // D layout: lane l holds D[4 (l / 16) + i][l % 16] (token, group column)
   const gemv_f32x4_t acc = acc0 + acc1;
 #pragma unroll
@@ -285,9 +285,9 @@ bool gemv_ok(int64_t tokens, int64_t k, int64_t n, int64_t hd, bool qk_norm, con
 }
 
 template <int TM>
-static void launch_gemv_t(bool fold, unsigned grid, const GemvKArgs& c, hipStream_t s) {
-  if (fold) hipLaunchKernelGGL((qkv_gemv_kernel<TM, true>), dim3(grid), dim3(256), 0, s, c);
-  else hipLaunchKernelGGL((qkv_gemv_kernel<TM, false>), dim3(grid), dim3(256), 0, s, c);
+static void launch_gemv_t(bool fold, unsigned grid, const GemvKArgs& c, const AppendArgs& aa, hipStream_t s) {
+  if (fold) hipLaunchKernelGGL((qkv_gemv_kernel<TM, true>), dim3(grid), dim3(256), 0, s, c, aa);
+  else hipLaunchKernelGGL((qkv_gemv_kernel<TM, false>), dim3(grid), dim3(256), 0, s, c, aa);
 }
 
 void launch_qkv_gemv(GemvArgs d, bool fold, const QkvEpi& e, hipStream_t s) {
@@ -301,7 +301,7 @@ void launch_qkv_gemv(GemvArgs d, bool fold, const QkvEpi& e, hipStream_t s) {
   GemvKArgs c{};
   c.a = d.a; c.w = d.w; c.gamma = d.gamma;
   c.bias = e.bias; c.positions = e.positions; c.cs = e.cs;
-  c.out = e.out; c.status = e.status; c.cache = e.cache; c.slot_off = e.slot_off;
+  c.out = e.out; c.status = e.status; c.cache = e.cache;
   c.ldo = e.ldo; c.c_skv = e.c_skv; c.c_sh = e.c_sh;
   c.m = static_cast<int32_t>(d.m); c.k = static_cast<int32_t>(d.k);
   c.lda = static_cast<int32_t>(d.lda); c.ldw = static_cast<int32_t>(d.ldw); c.pw = static_cast<int32_t>(pg);
@@ -312,10 +312,10 @@ void launch_qkv_gemv(GemvArgs d, bool fold, const QkvEpi& e, hipStream_t s) {
   c.bias_dt = static_cast<uint8_t>(e.bias_dtype); c.qkv_dt = static_cast<uint8_t>(e.qkv_dt);
   c.out_dt = static_cast<uint8_t>(e.out_dt); c.cache_dt = static_cast<uint8_t>(e.cache_dt);
   c.pos_is_i64 = static_cast<uint8_t>(e.pos_is_i64); c.skip_kv_out = static_cast<uint8_t>(e.skip_kv_out);
-  if (d.m <= 1) launch_gemv_t<1>(fold, grid, c, s);
-  else if (d.m <= 2) launch_gemv_t<2>(fold, grid, c, s);
-  else if (d.m <= 4) launch_gemv_t<4>(fold, grid, c, s);
-  else launch_gemv_t<8>(fold, grid, c, s);
+  if (d.m <= 1) launch_gemv_t<1>(fold, grid, c, e.app, s);
+  else if (d.m <= 2) launch_gemv_t<2>(fold, grid, c, e.app, s);
+  else if (d.m <= 4) launch_gemv_t<4>(fold, grid, c, e.app, s);
+  else launch_gemv_t<8>(fold, grid, c, e.app, s);
 }
 
 }  // namespace bfa

@@ -375,7 +375,7 @@ int bfa_append_paged_kv(const void* k, const void* v, int kv_dtype, int64_t num_
  * write_kv_out = 0 leaves the k/v columns of out unwritten (q only).  Cache
  * strides must be multiples of 4 elements and the cache 16-byte aligned.
  * workspace: bfa_fused_rmsnorm_qkv_append_workspace_size() bytes (the fused
- * workspace plus tokens x 8 bytes of resolved cache slots). */
+ * workspace plus tokens x 8 bytes). */
 int64_t bfa_fused_rmsnorm_qkv_append_workspace_size(int64_t tokens, int64_t hidden,
                                                     int64_t qkv_dim, int64_t head_dim);
 int bfa_fused_rmsnorm_qkv_append(
