@@ -10,6 +10,8 @@ the library is missing, or a tensor is not on a ROCm device, the call raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import threading
 import warnings
 from ctypes import c_float, c_int, c_int64, c_void_p
@@ -149,21 +151,38 @@ def exported_symbols():
     return list(_SIGNATURES)
 
 
+_entries = None  # the module of vector-call entry points (csrc/pyentry.cpp)
+
+
+def _load_entries():
+    global _entries
+    load()  # the library first: one copy serves both, and its absence is reported there
+    with _lock:
+        if _entries is None:
+            path = LIB_PATH.parent / "_bfa_entry.so"
+            if not path.exists():
+                raise RuntimeError(
+                    f"braidinfer_amd entry module not found at {path}; "
+                    "build it with `python -m braidinfer_amd.build`")
+            loader = importlib.machinery.ExtensionFileLoader("_bfa_entry", str(path))
+            mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_bfa_entry", loader))
+            loader.exec_module(mod)
+            _entries = mod
+    return _entries
+
+
 def call(name: str, *args) -> int:
     """Calls entry point `name`; raises BraidinferAMDError on a negative return."""
-    lib = load()
-    rc = getattr(lib, name)(*args)
-    if name.endswith("workspace_size"):
-        return rc
-    if rc < 0:
+    rc = getattr(_entries or _load_entries(), name)(*args)
+    if rc < 0 and not name.endswith("workspace_size"):
         raise_error(rc)
     return rc
 
 
 def entry(name: str):
-    """The bound ctypes function of entry point `name`, for hot paths that call
-    it directly and pass a negative return code to raise_error()."""
-    return getattr(load(), name)
+    """The bound function of entry point `name`, for hot paths that call it
+    directly and pass a negative return code to raise_error()."""
+    return getattr(_entries or _load_entries(), name)
 
 
 def raise_error(rc: int) -> None:
@@ -176,7 +195,7 @@ def raise_error(rc: int) -> None:
 def workspace_size(name: str, *args) -> int:
     """`<name>(*args)` of a workspace-size entry point (not memoised: the plan
     it reflects also follows the planner overrides, see set_tuning)."""
-    return getattr(load(), name)(*args)
+    return getattr(_entries or _load_entries(), name)(*args)
 
 
 # Planner overrides (BFA_TUNE_* of include/braidinfer_amd.h).  The library reads
@@ -251,11 +270,11 @@ def clear_workspaces(device: torch.device | int | None = None) -> int:
 
 
 def dtype_code(t: torch.Tensor | torch.dtype) -> int:
-    dt = t if isinstance(t, torch.dtype) else t.dtype
-    try:
-        return _DTYPE_CODE[dt]
-    except KeyError:
-        raise TypeError(f"braidinfer_amd: unsupported dtype {dt}") from None
+    dt = t if type(t) is torch.dtype else t.dtype
+    code = _DTYPE_CODE.get(dt)
+    if code is None:
+        raise TypeError(f"braidinfer_amd: unsupported dtype {dt}")
+    return code
 
 
 def ptr(t: torch.Tensor | None):

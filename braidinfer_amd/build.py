@@ -4,7 +4,8 @@ Usage:  python -m braidinfer_amd.build [--jobs N]
 
 Every ``csrc/*.hip`` file is compiled to an object in parallel, then linked
 into ``braidinfer_amd/lib/libbraidinfer_amd.so``.  The library is the product:
-the Python package loads it with ctypes and fails loudly when it is missing.
+the Python package loads it and fails loudly when it is missing.  The package's
+own calls go through ``lib/_bfa_entry.so`` (csrc/pyentry.cpp).
 """
 from __future__ import annotations
 
@@ -14,6 +15,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -23,6 +25,7 @@ INCLUDE = ROOT / "include"
 LIBDIR = PKG / "lib"
 OBJDIR = LIBDIR / "obj"
 LIBNAME = "libbraidinfer_amd.so"
+ENTRYNAME = "_bfa_entry.so"
 ARCH = "gfx950"
 
 # -ffp-contract=off keeps every product and sum separately rounded, the way the
@@ -58,6 +61,19 @@ def _compile(src: Path) -> Path:
     return obj
 
 
+def _build_entry() -> Path:
+    """The CPython module over the library (csrc/pyentry.cpp), next to it."""
+    tmp = LIBDIR / (ENTRYNAME + ".tmp")
+    cmd = [hipcc(), "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-Wall", f"-I{INCLUDE}",
+           f"-I{sysconfig.get_paths()['include']}", str(CSRC / "pyentry.cpp"), "-shared", f"-L{LIBDIR}",
+           f"-l:{LIBNAME}", "-Wl,-rpath,$ORIGIN", "-o", str(tmp)]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"building {ENTRYNAME} failed:\n{proc.stdout}\n{proc.stderr}")
+    os.replace(tmp, LIBDIR / ENTRYNAME)
+    return LIBDIR / ENTRYNAME
+
+
 def build(jobs: int | None = None, verbose: bool = False) -> Path:
     """Compiles every csrc/*.hip file and links the shared library; returns its path."""
     OBJDIR.mkdir(parents=True, exist_ok=True)
@@ -74,6 +90,7 @@ def build(jobs: int | None = None, verbose: bool = False) -> Path:
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stdout}\n{proc.stderr}")
     os.replace(tmp, out)
+    _build_entry()
     if verbose:
         print(f"built {out}")
     return out

@@ -265,6 +265,6 @@ def split_heads(output: torch.Tensor, num_q_heads: int, num_kv_heads: int):
     (the split/view sequence of the reference variants)."""
     tokens, qkv_dim = output.shape
     hd = head_dim_of(qkv_dim, num_q_heads, num_kv_heads)
-    q, k, v = output.split([num_q_heads * hd, num_kv_heads * hd, num_kv_heads * hd], dim=-1)
+    q, k, v = output.split_with_sizes([num_q_heads * hd, num_kv_heads * hd, num_kv_heads * hd], -1)
     return (q.view(tokens, num_q_heads, hd), k.view(tokens, num_kv_heads, hd),
             v.view(tokens, num_kv_heads, hd))

@@ -167,28 +167,41 @@ class PagedKVAppend:
             raise ZeroDivisionError("integer division or modulo by zero")
         if self.page_size < 0:
             raise ValueError("page_size must be positive")
-        positions = self.positions.reshape(-1)
-        if positions.numel() < num_tokens:
-            raise IndexError(f"{positions.numel()} positions for {num_tokens} tokens")
-        positions = positions[:num_tokens]
+        positions = self.positions
+        if positions.dim() != 1:
+            positions = positions.reshape(-1)
+        given = positions.numel()
+        if given < num_tokens:
+            raise IndexError(f"{given} positions for {num_tokens} tokens")
+        if given != num_tokens:
+            positions = positions[:num_tokens]
         if positions.dtype not in (torch.int32, torch.int64):
             positions = positions.long()
-        if self.kv_indices.dim() > 1:
+        kv_indices = self.kv_indices
+        if kv_indices.dim() > 1:
             raise ValueError("kv_indices must be one-dimensional")
-        kv_indices = self.kv_indices.reshape(-1)
+        if kv_indices.dim() != 1:
+            kv_indices = kv_indices.reshape(-1)
         if kv_indices.dtype not in (torch.int32, torch.int64):
             kv_indices = kv_indices.long()
         kv_indptr = batch_indices = None
         if self.kv_indptr is not None:
             if self.batch_indices is None:
                 raise ValueError("a batched append needs batch_indices")
-            kv_indptr = self.kv_indptr.reshape(-1).to(torch.int32).contiguous()
-            batch_indices = self.batch_indices.reshape(-1)
+            kv_indptr = self.kv_indptr
+            if kv_indptr.dim() != 1 or kv_indptr.dtype != torch.int32 or not kv_indptr.is_contiguous():
+                kv_indptr = kv_indptr.reshape(-1).to(torch.int32).contiguous()
+            batch_indices = self.batch_indices
+            if batch_indices.dim() != 1:
+                batch_indices = batch_indices.reshape(-1)
             if batch_indices.dtype not in (torch.int32, torch.int64):
                 batch_indices = batch_indices.long()
-            if batch_indices.numel() < num_tokens:
-                raise IndexError(f"{batch_indices.numel()} batch indices for {num_tokens} tokens")
-            batch_indices = batch_indices[:num_tokens].contiguous()
+            given = batch_indices.numel()
+            if given < num_tokens:
+                raise IndexError(f"{given} batch indices for {num_tokens} tokens")
+            if given != num_tokens:
+                batch_indices = batch_indices[:num_tokens]
+            batch_indices = batch_indices.contiguous()
         # keep the converted tensors alive until the call has been queued
         self._keep = (positions.contiguous(), kv_indices.contiguous(), kv_indptr, batch_indices)
         positions, kv_indices = self._keep[0], self._keep[1]

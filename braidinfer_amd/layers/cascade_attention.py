@@ -149,10 +149,13 @@ class CascadeAttention:
             kn_w = kn_w.contiguous()
             kn_dt = _lib.dtype_code(kn_w)
             kn_eps = float(getattr(k_norm, "eps", getattr(k_norm, "variance_epsilon", 1e-6)))
-        qpos = query_positions.reshape(-1)
-        if qpos.numel() < tokens:
-            raise IndexError(f"{qpos.numel()} query positions for {tokens} tokens")
-        qpos = qpos[:tokens].contiguous()
+        qpos = query_positions if query_positions.dim() == 1 else query_positions.reshape(-1)
+        given = qpos.numel()
+        if given < tokens:
+            raise IndexError(f"{given} query positions for {tokens} tokens")
+        if given != tokens:
+            qpos = qpos[:tokens]
+        qpos = qpos.contiguous()
         if qpos.dtype not in (torch.int32, torch.int64):
             qpos = qpos.long()
         ws_bytes = _lib.workspace_size("bfa_cascade_attention_workspace_size", tokens, self.num_heads, hkv, d,
@@ -161,13 +164,13 @@ class CascadeAttention:
         st = kv_cache.stride()
         _lib.call(
             "bfa_cascade_attention",
-            _lib.ptr(query), _lib.dtype_code(query), tokens, self.num_heads,
-            query.stride(0), query.stride(1), _lib.ptr(qpos), _lib.dtype_code(qpos),
-            _lib.ptr(kv_cache), num_pages, hkv, self.page_size, d, st[0], st[1], st[2], st[3],
+            query.data_ptr(), _lib.dtype_code(query), tokens, self.num_heads,
+            query.stride(0), query.stride(1), qpos.data_ptr(), _lib.dtype_code(qpos),
+            kv_cache.data_ptr(), num_pages, hkv, self.page_size, d, st[0], st[1], st[2], st[3],
             entries, _lib.ptr(e_page), _lib.ptr(e_kstart), _lib.ptr(e_delta), _lib.ptr(e_info),
             _lib.ptr(cs), max_pos, _lib.ptr(kn_w), kn_dt, kn_eps,
-            float(self.scale), int(bool(causal_mask)), _lib.ptr(out), out.stride(0),
-            _lib.ptr(ws), ws.numel(), _lib.ptr(_lib.status_word(dev)), _lib.stream_of(dev),
+            float(self.scale), int(bool(causal_mask)), out.data_ptr(), hd,
+            ws.data_ptr(), ws.numel(), _lib.status_word(dev).data_ptr(), _lib.stream_of(dev),
         )
         return out
 
@@ -179,16 +182,19 @@ class CascadeAttention:
         position by their kv_length.  flags bit 0: attended, bit 1: K is rotated
         (a rotary table, a global_position_start and a nonzero delta, :148-170)."""
         meta, cumulative = [], 0
+        rotates = 2 if self.rotary_emb is not None else 0
         for level in cascade_levels:
             for chunk in level.chunks:
-                attended = bool(chunk.page_table) and chunk.kv_length != 0
                 cached = getattr(chunk, "cached_position_start", 0)
-                glob = getattr(chunk, "global_position_start", cached)
-                delta = glob - cached
-                rotate = self.rotary_emb is not None and hasattr(chunk, "global_position_start") and delta != 0
-                meta.append((delta, cumulative, int(attended) | (int(rotate) << 1)))
-                if attended:
-                    cumulative += chunk.kv_length
+                # (without a global position the delta is 0, so K is not rotated)
+                delta = getattr(chunk, "global_position_start", cached) - cached
+                flags = rotates if delta != 0 else 0
+                length = chunk.kv_length
+                if chunk.page_table and length != 0:
+                    meta.append((delta, cumulative, flags | 1))
+                    cumulative += length
+                else:
+                    meta.append((delta, cumulative, flags))
         return meta
 
     def _plan(self, cascade_levels, meta, dev):

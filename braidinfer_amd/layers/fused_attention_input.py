@@ -25,7 +25,7 @@ from ..kernels._qkv import fused_rmsnorm_qkv, head_dim_of
 
 def _split_flat(out: torch.Tensor, num_heads: int, num_kv_heads: int):
     hd = head_dim_of(out.shape[1], num_heads, num_kv_heads)
-    return out.split([num_heads * hd, num_kv_heads * hd, num_kv_heads * hd], dim=-1)
+    return out.split_with_sizes([num_heads * hd, num_kv_heads * hd, num_kv_heads * hd], -1)
 
 
 def qwen3_attention_input(hidden_states: torch.Tensor, layernorm_weight: torch.Tensor,

@@ -30,7 +30,7 @@ def _rows(x: torch.Tensor, k: int) -> torch.Tensor:
     row stride (a copy only when the view does not qualify)."""
     if x.shape[-1] != k:
         raise ValueError(f"input has {x.shape[-1]} features, the layer takes {k}")
-    x2 = x.reshape(-1, k)
+    x2 = x if x.dim() == 2 else x.reshape(-1, k)
     if x2.stride(-1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16:
         x2 = x2.contiguous()
     return x2
@@ -60,7 +60,7 @@ def _run(x: torch.Tensor, weight: torch.Tensor, n: int, mode: int, bias=None, re
     if residual is not None:
         if residual.shape[-1] != n or residual.numel() != tokens * n:
             raise ValueError(f"residual of shape {tuple(residual.shape)} does not match [{tokens}, {n}]")
-        r2 = residual.reshape(tokens, n)
+        r2 = residual if residual.dim() == 2 else residual.reshape(tokens, n)
         if r2.stride(-1) != 1:
             r2 = r2.contiguous()
     if bias is not None:
@@ -68,16 +68,17 @@ def _run(x: torch.Tensor, weight: torch.Tensor, n: int, mode: int, bias=None, re
             raise ValueError(f"bias has {bias.numel()} elements, the layer has {n} outputs")
         bias = bias.detach().contiguous()
     ws_bytes = _lib.workspace_size("bfa_linear_workspace_size", tokens, k, n, mode)
-    ws = _lib.workspace(dev, ws_bytes)
+    ws = _lib.workspace(dev, ws_bytes) if ws_bytes else None
+    code = _lib.dtype_code(x2)
     _lib.call(
-        "bfa_linear", _lib.ptr(x2), _lib.dtype_code(x2), tokens, k, x2.stride(0),
-        _lib.ptr(weight), n, weight.stride(0), _lib.ptr(bias),
+        "bfa_linear", x2.data_ptr(), code, tokens, k, x2.stride(0),
+        weight.data_ptr(), n, weight.stride(0), _lib.ptr(bias),
         _lib.dtype_code(bias) if bias is not None else 0, mode,
-        _lib.dtype_code(x2) if proj_dtype is None else proj_dtype,
+        code if proj_dtype is None else proj_dtype,
         _lib.ptr(r2), _lib.dtype_code(r2) if r2 is not None else 0, r2.stride(0) if r2 is not None else n,
-        sum_dtype, _lib.ptr(out), _lib.dtype_code(out), out.stride(0), _lib.ptr(ws), ws.numel(),
-        _lib.stream_of(dev))
-    return out.view(*x.shape[:-1], n)
+        sum_dtype, out.data_ptr(), code if out_t == x2.dtype else _lib.dtype_code(out), n,
+        None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _lib.stream_of(dev))
+    return out if x.dim() == 2 else out.view(*x.shape[:-1], n)
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
