@@ -1,7 +1,8 @@
 // CPython module _bfa_entry: the C ABI's entry points as vector-call functions.
 //
 // Each entry takes the C function's arguments in order: int for int and int64_t,
-// int or None for pointers, a number for float; it returns the C result.  ctypes
+// int or None for pointers, a number for float (or a ctypes scalar of these); it
+// returns the C result.  ctypes
 // converts the 50 arguments of a fused call through Python-level argument types in
 // about 5 us, as long as two kernel launches; these functions take 1.
 #define PY_SSIZE_T_CLEAN
@@ -18,6 +19,17 @@ namespace {
 
 template <class T>
 bool from_py(PyObject* o, T& v) {
+  if (!PyLong_Check(o) && !PyFloat_Check(o) && o != Py_None) {
+    // a ctypes scalar (c_void_p, c_float, ...) stands for its value
+    if (PyObject* value = PyObject_GetAttrString(o, "value")) {
+      const bool plain = PyLong_Check(value) || PyFloat_Check(value) || value == Py_None;
+      const bool ok = plain && from_py(value, v);
+      if (!plain) PyErr_SetString(PyExc_TypeError, "an int, a float, None or a ctypes scalar is required");
+      Py_DECREF(value);
+      return ok;
+    }
+    PyErr_Clear();
+  }
   if constexpr (std::is_pointer_v<T>) {
     if (o == Py_None) {
       v = nullptr;

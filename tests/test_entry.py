@@ -3,6 +3,8 @@ that returns a number, the same results as through ctypes, and argument errors
 raised before the call."""
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 
 from braidinfer_amd import _lib
@@ -31,4 +33,4 @@ def test_errors_and_their_text():
         fn("0")
     with pytest.raises(OverflowError):
         fn(1 << 40)
-    assert fn(0) == -1
+    assert fn(0) == -1 and fn(ctypes.c_int(0)) == -1
