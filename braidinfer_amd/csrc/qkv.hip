@@ -394,11 +394,11 @@ __device__ __forceinline__ void tile_origin(const GemmArgs& g, int64_t tile, int
 // per wave, requested before the K loop).  SLOT_U4: uint4 offset in lds of the
 // fused KV append's slot table (MB x 32 int64 per wave), followed by the row
 // scales' table (MB x 32 floats per wave).
-template <int EPI, int HD, int MB, int NB, int WM, int WN, int NW, int EDT, bool EARLY, int SLOT_U4, typename ACC>
+template <int EPI, int HD, int MB, int NB, int WM, int WN, int NW, bool EARLY, int SLOT_U4, typename ACC>
 __device__ __forceinline__ void gemm_epilogue(ACC& acc, uint4* lds, const GemmArgs& g, const QkvEpi& e,
                                               int64_t m0, int64_t n0, int wid, int wm, int wn, int lane,
                                               const int64_t* praw) {
-  using DT = QkvDt<EDT>;
+  using DT = QkvDt<EDT_RT>;  // the shapes with compiled-in dtypes are qkv_prefill.hip's
   constexpr bool A16 = sizeof(acc[0][0]) == sizeof(f32x4_t);  // 16x16 accumulator blocks
   constexpr int LDR = 136;
   constexpr bool EARLY_POS = EARLY;
@@ -725,8 +725,7 @@ __device__ __forceinline__ void gemm_epilogue(ACC& acc, uint4* lds, const GemmAr
 // 4-wave workgroups, or one 8-wave workgroup, per CU.  BK is the depth of a DMA
 // stage: 32 (ring of NS stages, 16 rows x 64 bytes per copy) or 64 (two
 // buffers, 8 rows x 128 bytes per copy, full cache lines).
-template <int BM, int BN, int WM, int WN, bool BF16, int EPI, int HD, bool DIRECT, int NS, int BK,
-          int EDT = EDT_RT>
+template <int BM, int BN, int WM, int WN, bool BF16, int EPI, int HD, bool DIRECT, int NS, int BK>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, (WM * WN <= 8192 ? 2 : 1)) void qkv_gemm_kernel(
     GemmArgs g, QkvEpi e) {
   constexpr int NWN = BN / WN;
@@ -815,11 +814,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, (WM * WN <= 8192 ? 2 : 
   // v_mfma_f32_32x32x16 into 32x32 blocks (acc).  Same product and the same
   // fragment bytes per wave tile, but a 16x16x32 MFMA reads and writes a quarter
   // of the accumulators for half the work, and the chip is power limited under
-  // this loop: at 8192 tokens the Llama-3-8B projection took 313-325 against
-  // 323-334 us and the fused op 329-334 against 344-347 us, same box,
-  // interleaved processes; with the pinned loop below, gate_up+SiLU*mul
-  // 1560-1568 against 1605-1613 us, down_proj+residual 777-778 against 810-812
-  // us and o_proj+residual 230-232 against 233 us (the 32x32x16 loop pinned).
+  // this loop.
   constexpr bool M16 = DIRECT && BK == 64;
   f32x16_t acc[M16 ? 1 : MB][M16 ? 1 : NB];
   f32x4_t acc4[M16 ? 2 * MB : 1][M16 ? 2 * NB : 1];
@@ -1006,10 +1001,10 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, (WM * WN <= 8192 ? 2 : 
   int lane_e = lane, wid_e = wid;
   if constexpr (PERSIST) asm volatile("" : "+v"(lane_e), "+s"(wid_e));
   if constexpr (M16)
-    gemm_epilogue<EPI, HD, MB, NB, WM, WN, NW, EDT, EARLY_POS, SLOT_U4>(acc4, lds, g, e, m0, n0, wid_e,
+    gemm_epilogue<EPI, HD, MB, NB, WM, WN, NW, EARLY_POS, SLOT_U4>(acc4, lds, g, e, m0, n0, wid_e,
                                                                       wid_e / NWN, wid_e % NWN, lane_e, praw);
   else
-    gemm_epilogue<EPI, HD, MB, NB, WM, WN, NW, EDT, EARLY_POS, SLOT_U4>(acc, lds, g, e, m0, n0, wid_e,
+    gemm_epilogue<EPI, HD, MB, NB, WM, WN, NW, EARLY_POS, SLOT_U4>(acc, lds, g, e, m0, n0, wid_e,
                                                                       wid_e / NWN, wid_e % NWN, lane_e, praw);
   if constexpr (!PERSIST) break;  // one tile per workgroup: no loop, nothing hoisted out of one
   }
@@ -2617,10 +2612,8 @@ static int fused_edt(const QkvEpi& e) {
 
 // Workgroups of a prefill GEMM launch: one per tile, or for the 256x256 tile
 // (one workgroup per CU, the kernel's PERSIST form) one per CU, each looping
-// over tiles: the Llama-3-8B projection at 8192 tokens (768 tiles) took 380.5
-// against 388.0 us on one box, with bit-identical output.  Planner override
-// BFA_TUNE_QKV_PERSIST = c sets the workgroups per CU of the 256x256 tile
-// (0: one per tile).
+// over tiles.  Planner override BFA_TUNE_QKV_PERSIST = c sets the workgroups per
+// CU of the 256x256 tile (0: one per tile).
 static unsigned persistent_grid(int64_t tiles, bool persist) {
   int per_cu = persist ? 1 : 0;
   const int c = tuning(BFA_TUNE_QKV_PERSIST);
