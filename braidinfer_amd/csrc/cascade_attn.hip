@@ -653,17 +653,18 @@ __device__ __forceinline__ int kslot(int r, int gr) {
 // One wave takes RB blocks of 16 query rows, so a K or V^T fragment read from the
 // LDS feeds RB MFMAs.  With RB = 1 the loop is bound by those reads (32 KiB per
 // wave and tile, 2000 LDS cycles per CU against 1024 of MFMA) and by the softmax's
-// VALU work; RB = 2 halves the first, and per score the second is a maximum, one
-// multiply-add, the exponential, the sum and half a conversion:
-//   * tiles whose keys every row of the wave may see skip the masking (one
-//     compare per lane; a tile with the unused slots of a page, or at the causal
-//     edge, takes it);
-//   * the scale goes into the exponential's argument.
+// VALU work; RB = 2 halves the first, and tiles whose keys every row of the wave
+// may see skip the masking (one compare per lane; a tile with the unused slots of
+// a page, or at the causal edge, takes it).
+// The score is scaled, then masked, then the maximum is taken from it: as one
+// multiply-add, s * scale - max, the exponential's argument kept the rounding
+// error of max (128 and more from scores of 2^31: p overflowed) and made NaN of a
+// masked score at scale 0.  The two operations cost 115 -> 117 us of the call below.
 // The running maximum follows every larger score: letting it lag by up to 2^8
-// saved rescalings (124 against 129 us for the call below) but rounded the largest p, exactly 1
+// saved rescalings (124 against 129 us) but rounded the largest p, exactly 1
 // otherwise, and the error against 64 bits rose from 0.0069 to 0.0070.
-// Qwen3 shape, 1000 queries over 9000 keys: the call 197 -> 129 us (this kernel
-// 176 -> 104 us, 670 TFLOP/s of attended pairs); Llama-3-8B 333 -> 212 us.
+// Graph-replayed calls against one block per wave: Qwen3 shape, 1000 queries over
+// 9000 keys, 172 -> 117 us (this kernel 102 us); Llama-3-8B 317 -> 205 us.
 // Moving the exponentials of one tile between the MFMAs of the next tile's scores
 // (two score sets) was slower, 126 against 123 us, and so were raised wave
 // priorities around the products (126 against 124 us).
@@ -777,8 +778,14 @@ __global__ __launch_bounds__(256, 2) void cascade_flat_kernel(CasArgs a, FlatArg
           for (int rb = 0; rb < RB; ++rb) s[rb][c] = mfma16x32<BF16>(kf, qf[rb][j], s[rb][c]);
         }
     };
-    auto mask = [&](int32_t kp, cas_f32x4_t (&s)[RB][4]) {
-      if (!__any(kp > qmin)) return;
+    // times the scale, then masked: a masked score is -inf whatever the scale
+    auto weigh = [&](int32_t kp, cas_f32x4_t (&s)[RB][4]) {
+      const bool edge = __any(kp > qmin);
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) s[rb][c] *= sl2;
+      if (!edge) return;
 #pragma unroll
       for (int c = 0; c < 4; ++c)
 #pragma unroll
@@ -797,7 +804,7 @@ __global__ __launch_bounds__(256, 2) void cascade_flat_kernel(CasArgs a, FlatArg
       return mx;
     };
     auto new_max = [&](int rb, float mx) {
-      mx = lanes4_max(mx) * sl2;
+      mx = lanes4_max(mx);
       if (!__any(mx > m[rb])) return;
       const float m_new = fmaxf(m[rb], mx);
       const float alpha = __builtin_amdgcn_exp2f(m[rb] - (m_new == -INFINITY ? 0.f : m_new));
@@ -826,7 +833,7 @@ __global__ __launch_bounds__(256, 2) void cascade_flat_kernel(CasArgs a, FlatArg
       }
       if (!__all(kp > qmax)) {  // (all: no row of the wave sees a key of the tile)
         scores(kbuf[b], sc);
-        mask(kp, sc);
+        weigh(kp, sc);
         uint4 pf[RB][2];
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
@@ -837,10 +844,10 @@ __global__ __launch_bounds__(256, 2) void cascade_flat_kernel(CasArgs a, FlatArg
           for (int c = 0; c < 4; ++c)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              sc[rb][c][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[rb][c][i], sl2, -mref));
+              sc[rb][c][i] = __builtin_amdgcn_exp2f(sc[rb][c][i] - mref);
               rs += sc[rb][c][i];
             }
-          l[rb] += rs;  // this lane's keys; the lanes of a row meet at the end
+          l[rb] += rs;
 #pragma unroll
           for (int h = 0; h < 2; ++h)
             pf[rb][h] = make_uint4(pack_pair<BF16>(sc[rb][2 * h][0], sc[rb][2 * h][1]),
@@ -868,12 +875,12 @@ __global__ __launch_bounds__(256, 2) void cascade_flat_kernel(CasArgs a, FlatArg
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     const int64_t r = row0 + 16 * rb + (lane & 15);
-    const float ls = lanes4_sum(l[rb]);
+    l[rb] = lanes4_sum(l[rb]);
     if (r >= rows) continue;
     const int d0 = 4 * (lane >> 4);
     if (gridDim.z == 1) {
       const int64_t t = r / a.group, hh = g * a.group + (r - t * a.group);
-      const float inv = 1.0f / fmaxf(ls, 1e-12f);
+      const float inv = 1.0f / fmaxf(l[rb], 1e-12f);
       uint16_t* orow = static_cast<uint16_t*>(a.out) + t * a.out_st + hh * D;
 #pragma unroll
       for (int j = 0; j < OJ; ++j)
@@ -884,7 +891,7 @@ __global__ __launch_bounds__(256, 2) void cascade_flat_kernel(CasArgs a, FlatArg
       float* pr = a.part + ((static_cast<int64_t>(blockIdx.z) * a.hkv + g) * rows + r) * (D + 2);
       if (lane < 16) {
         pr[0] = m[rb];
-        pr[1] = ls;
+        pr[1] = l[rb];
       }
 #pragma unroll
       for (int j = 0; j < OJ; ++j)

@@ -1,7 +1,8 @@
 """The flat form of cascade attention at the edges of its row blocks: one and two
 16-row blocks per wave (from 257 rows per kv head at head_dim 128, 1025 at 64),
 against the oracle; and what its softmax does with scores that keep growing
-along the keys and with a negative scale, against 64 bits."""
+along the keys, with scores of 2^34, and with a negative or zero scale, against
+64 bits."""
 from __future__ import annotations
 
 import pytest
@@ -58,3 +59,52 @@ def test_growing_scores_and_sign(tuning, tokens, wg):
     hide = torch.arange(total)[None, :] > qpos[:, None]
     exp = torch.einsum("htk,khd->thd", torch.softmax(sc.masked_fill(hide, float("-inf")), -1), v)
     assert_close(outs[0].reshape(tokens, hq, d), exp, what=f"growing scores tokens={tokens} wg={wg}")
+
+
+@pytest.mark.parametrize("tokens", [100, 300])
+@pytest.mark.parametrize("causal", [True, False])
+def test_zero_scale(tuning, tokens, causal):
+    """Every score is 0: the mean of the visible values, with partly filled pages
+    and a causal edge inside a tile."""
+    tuning("CASCADE_FLAT", 1)
+    hq, hkv, d, ps = 8, 4, 128, 16
+    chunks, kv, total = build_case(93, hq, hkv, [130, 77, tokens], [0, 0, 0], pages=60)
+    q = randn(gen(94), tokens, hq, d)
+    qpos = torch.arange(total - tokens, total)
+    att = CascadeAttention(hq, d, 0.0, hkv, ps, rotary_emb=RotaryEmbedding(d, d, 4096, 1e6).to(DEV))
+    out = att.forward(q.to(DEV), qpos.to(DEV), kv.to(DEV), att.create_cascade_levels(chunks), 0, causal_mask=causal)
+    v = torch.cat([kv[c.page_table, 1].double().transpose(1, 2).reshape(-1, hkv, d)[: c.kv_length] for c in chunks])
+    seen = torch.arange(1, total + 1).view(-1, 1, 1)
+    mean = (v.cumsum(0) / seen)[qpos] if causal else v.mean(0, keepdim=True).expand(tokens, -1, -1)
+    assert_close(out.reshape(tokens, hq, d), mean.repeat_interleave(hq // hkv, 1), what=f"scale 0 causal={causal}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tokens", [100, 300])
+def test_scores_of_any_size(tuning, tokens, dtype):
+    """Scores up to 2^34 (2^28 in fp16), further apart than any exponential: each
+    query returns the value of its largest visible key."""
+    tuning("CASCADE_FLAT", 1)
+    hq, hkv, d, ps = 8, 4, 128, 16
+    chunks, kv, total = build_case(95, hq, hkv, [200, 90, tokens], [0, 0, 0], pages=60)
+    kv = kv.to(dtype)
+    g = gen(96)
+    sign = (torch.randint(0, 2, (d,), generator=g) * 2 - 1).to(dtype)
+    # keys of 128 sizes 1 to 2 apart by 2^-7, shuffled along the walk
+    size = 1 + torch.randint(0, 128, (total,), generator=g) / 128.0
+    big = 2.0 ** (15 if dtype == torch.bfloat16 else 12)
+    pos = 0
+    for c in chunks:
+        for j in range(c.kv_length):
+            kv[c.page_table[j // ps], 0, :, j % ps] = big * size[pos] * sign
+            pos += 1
+    q = (big * sign).expand(tokens, hq, d).contiguous()
+    qpos = torch.arange(total - tokens, total)
+    att = CascadeAttention(hq, d, d ** -0.5, hkv, ps, rotary_emb=RotaryEmbedding(d, d, 4096, 1e6).to(DEV))
+    out = att.forward(q.to(DEV), qpos.to(DEV), kv.to(DEV), att.create_cascade_levels(chunks), 0).cpu()
+    v = torch.cat([kv[c.page_table, 1].double().transpose(1, 2).reshape(-1, hkv, d)[: c.kv_length] for c in chunks])
+    exp = torch.empty(tokens, hkv, d, dtype=torch.float64)
+    for t in range(tokens):
+        seen = size[: int(qpos[t]) + 1]
+        exp[t] = v[: seen.numel()][seen == seen.max()].mean(0)  # equal keys share the weight
+    assert_close(out.reshape(tokens, hq, d), exp.repeat_interleave(hq // hkv, 1), what=f"scores of any size {dtype}")
