@@ -221,3 +221,17 @@ def test_fold_algebra_in_float64():
     assert torch.allclose(folded, ref, rtol=1e-12, atol=1e-12)
     wrong_axis = (x @ (w * gamma[:, None]).t()) * inv
     assert not torch.allclose(wrong_axis, ref, rtol=1e-3, atol=1e-3)
+
+
+def test_flat_attention_splits_down_to_one_tile(tuning):
+    """24 queries of TinyLlama (192 rows on 4 kv heads) over 127 pages: 32 tiles of
+    64 keys for fewer workgroups than CUs, so one tile per split.  The partials'
+    bytes (2 + head_dim floats per split, kv head and row) tell."""
+    from braidinfer_amd import _lib
+
+    def size():
+        return _lib.workspace_size("bfa_cascade_attention_workspace_size", 24, 32, 4, 64, 127, 16)
+
+    planned = size()
+    tuning("CASCADE_FLAT_WG", 1)  # one workgroup per block: unsplit
+    assert planned - size() == 32 * 4 * 192 * (64 + 2) * 4
