@@ -35,8 +35,9 @@ struct LinArgs {
 GemmPlan linear_plan(int64_t m, int64_t n, int64_t k, bool swiglu, bool split);
 void launch_linear_gemm(const GemmPlan& p, LinArgs q, int dt, hipStream_t st);
 
-// One launch, no workspace (of LinArgs: part and the planner's fields unused).
-bool linear_gemv_ok(int64_t m, int64_t wrows, int64_t k);
+// One launch, no workspace (of LinArgs: part and the planner's fields unused);
+// splits: of the split-K kernels for the same call.
+bool linear_gemv_ok(int64_t m, int64_t wrows, int64_t k, bool swiglu, int64_t splits);
 void launch_linear_gemv(LinArgs q, int dt, hipStream_t st);
 
 }  // namespace bfa

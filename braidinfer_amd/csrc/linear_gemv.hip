@@ -1,4 +1,5 @@
-// Linear layers of up to 16 tokens (64 for a small weight) in one launch:
+// Linear layers of up to 16 tokens (64 for a small weight) in one launch, where
+// that is faster than split-K (linear_gemv_ok):
 // y = x W^T with the layer's epilogue (bias, residual, or SiLU(gate) * up), 16-bit
 // operands, fp32 sums.
 //
@@ -189,22 +190,32 @@ void launch_form(const LinArgs& q, hipStream_t st) {
   hipLaunchKernelGGL((linear_gemv_kernel<DT, NWV, NR, MT, SWIGLU>), grid, dim3(NWV * 64), 0, st, q);
 }
 
-// Plain: one weight block, so that as many CUs as there are blocks of columns
-// stream (two blocks: Llama-3-8B down_proj at one token 24.9 -> 32.6 us), in 4
-// waves, 8 for a long K.  SwiGLU has twice the rows: two blocks, which halve the
-// token reads per weight byte (gate_up at 16 tokens 60.9 -> 48.7 us), but one for
-// up to 4 tokens of a weight of 32 MiB and more (41.3 against 42.7 us).
+// Waves and weight blocks of a workgroup.  Plain: one weight block, so that as many
+// CUs as there are blocks of columns stream (two blocks: Llama-3-8B down_proj at one
+// token 24.9 -> 32.6 us), in 4 waves, 8 for a long K and up to 16 tokens.  SwiGLU
+// has twice the rows: two blocks, which halve the token reads per weight byte
+// (gate_up at 16 tokens 60.9 -> 48.7 us), but one for up to 4 tokens of a weight of
+// 32 MiB and more (41.3 against 42.7 us).
+struct GemvForm {
+  int nwv, nr;
+};
+GemvForm gemv_form(int64_t m, int64_t n, int64_t k, bool swiglu) {
+  if (swiglu) return {4, m <= 4 && n * k * 4 >= (int64_t(32) << 20) ? 1 : 2};
+  return {m <= 16 && k >= 128 * 64 ? 8 : 4, 1};
+}
+
 template <int DT>
 void launch_dt(const LinArgs& q, hipStream_t st) {
   const int mt = static_cast<int>(cdiv(q.m, 16));
+  const GemvForm f = gemv_form(q.m, q.n, q.k, q.swiglu != 0);
   if (q.swiglu) {
-    if (q.m <= 4 && q.n * q.k * 4 >= (int64_t(32) << 20)) return launch_form<DT, 4, 1, 1, true>(q, st);
+    if (f.nr == 1) return launch_form<DT, 4, 1, 1, true>(q, st);
     if (mt == 1) return launch_form<DT, 4, 2, 1, true>(q, st);
     if (mt == 2) return launch_form<DT, 4, 2, 2, true>(q, st);
     if (mt == 3) return launch_form<DT, 4, 2, 3, true>(q, st);
     return launch_form<DT, 4, 2, 4, true>(q, st);
   }
-  if (mt == 1 && q.kt >= 128) return launch_form<DT, 8, 1, 1, false>(q, st);
+  if (f.nwv == 8) return launch_form<DT, 8, 1, 1, false>(q, st);
   if (mt == 1) return launch_form<DT, 4, 1, 1, false>(q, st);
   if (mt == 2) return launch_form<DT, 4, 1, 2, false>(q, st);
   if (mt == 3) return launch_form<DT, 4, 1, 3, false>(q, st);
@@ -213,18 +224,43 @@ void launch_dt(const LinArgs& q, hipStream_t st) {
 
 }  // namespace
 
-// Up to 16 tokens always; up to 64 while the weight is at most 16 MiB: above, a
-// workgroup's reads of all the tokens cost more than the split-K kernels' second
-// launch (24 tokens: TinyLlama down_proj, 23 MB, 16.6 against 14.8 us; o_proj, 8
-// MB, 8.5 against 10.4).  Overrides: BFA_TUNE_LINEAR_GEMV, and any of the split-K
-// kernels' own keeps them.
-bool linear_gemv_ok(int64_t m, int64_t wrows, int64_t k) {
+// Neither kernel is always ahead: a workgroup walks the whole of K, so a long K on
+// few columns leaves most CUs idle (1 token, K 65536, 128 columns 74 against 44 us
+// split; 64 tokens, K 8192, 1024 columns 39 against 17), and from some thousand
+// workgroups their start costs more than their stream (K 1024, 128256 columns 69
+// against 47 us).  So both times are estimated, in us, from what was measured of
+// either on 2753 shapes (1 to 64 tokens, K 64 to 65536, 16 to 128256 columns):
+//   here   3 + the longer of one workgroup's K steps and a CU's share of all of
+//          them; a step takes 0.31 at one token and 0.0125 more for each other
+//   split  5.4 (6 from 17 tokens) + 0.14 (0.083) per split that the reduction
+//          reads, 1.7 times that with SwiGLU, + the weight at 5.6 (6.9) TB/s, the
+//          partials' round trip and the outputs
+// each within 10 % for 8 in 10 shapes.  On those shapes the choice is within 3 % of
+// the faster one or ahead of split-K in all but one in ninety, 20 % behind at worst
+// (always taking this kernel up to 16 tokens, and up to 64 for 16 MiB, was behind
+// in one of three, by up to 8 times).
+// From 17 tokens only weights of up to 16 MiB are weighed.  Overrides:
+// BFA_TUNE_LINEAR_GEMV, and any of the split-K kernels' own keeps them.
+bool linear_gemv_ok(int64_t m, int64_t wrows, int64_t k, bool swiglu, int64_t splits) {
   if (m > 64 || k % 64 != 0) return false;
   const int o = tuning(BFA_TUNE_LINEAR_GEMV);
   if (o >= 0) return o != 0;
   if (tuning(BFA_TUNE_DECODE_KS) >= 0 || tuning(BFA_TUNE_DECODE_WG) >= 0 || tuning(BFA_TUNE_DECODE_SPLITS) >= 0)
     return false;
-  return m <= 16 || wrows * k * 2 <= (int64_t(16) << 20);
+  const double mb = static_cast<double>(wrows) * k * 2e-6, outs = static_cast<double>(m) * wrows * 1e-6;
+  if (m > 16 && wrows * k * 2 > (int64_t(16) << 20)) return false;
+  const int64_t n = swiglu ? wrows / 2 : wrows;
+  const GemvForm f = gemv_form(m, n, k, swiglu);
+  const double steps = static_cast<double>(cdiv(k / 64, f.nwv));
+  const int64_t wgs = cdiv(n, swiglu ? 8 * f.nr : 16);
+  const double cu = wgs > 256 ? static_cast<double>(cdiv(wgs, 256)) : static_cast<double>(wgs) / 256;  // per CU, at most
+  double step = 0.31 + 0.0125 * static_cast<double>(m - 1), busy = step;  // alone on a CU, with others
+  if (f.nr == 2) busy = step += 0.2;
+  if (f.nwv == 8) busy += 0.43, step *= 1.8;
+  const double here = 3 + std::max(steps * step, cu * ((m > 48 ? 1.7 : 0.7) + steps * busy));
+  const double sp = static_cast<double>(splits) * (swiglu ? 1.7 : 1);
+  const double split = m <= 16 ? 5.4 + 0.14 * sp + 0.18 * mb + 2.5 * outs : 6.0 + 0.083 * sp + 0.145 * mb + outs;
+  return here <= 0.965 * (split + 2.5 * static_cast<double>(splits) * outs);
 }
 
 void launch_linear_gemv(LinArgs q, int dt, hipStream_t st) {

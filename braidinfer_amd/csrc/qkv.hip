@@ -3278,13 +3278,14 @@ extern "C" int bfa_fused_rmsnorm_qkv_noalloc(
 // ------------------------------------------------------- linear fusions
 extern "C" int64_t bfa_linear_workspace_size(int64_t tokens, int64_t k, int64_t n, int mode) {
   if (tokens <= 0 || n <= 0) return 0;
-  const int64_t nw = mode == BFA_LINEAR_SILU_AND_MUL ? 2 * n : n;
-  if (linear_gemv_ok(tokens, nw, k)) return 0;
+  const bool swiglu = mode == BFA_LINEAR_SILU_AND_MUL;
+  const int64_t nw = swiglu ? 2 * n : n;
   const QkvPlan p = make_plan(tokens, nw, k, 0);
+  if (linear_gemv_ok(tokens, nw, k, swiglu, p.splits)) return 0;
   if (p.decode) return p.part_bytes;
   // above 64 tokens: the fp32 partials of the tiles that are split over K; a
   // caller without that workspace gets the plan without a split
-  return k % 64 == 0 ? linear_plan(tokens, n, k, mode == BFA_LINEAR_SILU_AND_MUL, true).part_bytes : 0;
+  return k % 64 == 0 ? linear_plan(tokens, n, k, swiglu, true).part_bytes : 0;
 }
 
 extern "C" int bfa_linear(const void* x, int dtype, int64_t tokens, int64_t k, int64_t x_stride,
@@ -3315,7 +3316,8 @@ extern "C" int bfa_linear(const void* x, int dtype, int64_t tokens, int64_t k, i
   const hipStream_t st = as_stream(stream);
   const bool vec = aligned16(out) && out_stride % 8 == 0 &&
                    (residual == nullptr || (aligned16(residual) && residual_stride % 8 == 0));
-  const bool gemv = linear_gemv_ok(tokens, nw, k);
+  const QkvPlan p = make_plan(tokens, nw, k, 0);
+  const bool gemv = linear_gemv_ok(tokens, nw, k, swiglu, p.splits);
   if (gemv || (tokens > 64 && k % 64 == 0 && tokens * x_stride * 2 < (int64_t(1) << 32) &&
                nw * w_stride * 2 < (int64_t(1) << 32))) {
     LinArgs q{};
@@ -3337,7 +3339,6 @@ extern "C" int bfa_linear(const void* x, int dtype, int64_t tokens, int64_t k, i
     launch_linear_gemm(lp, q, dtype, st);
     return check_launch(what);
   }
-  const QkvPlan p = make_plan(tokens, nw, k, 0);
   const int64_t need = p.decode ? p.part_bytes : 0;
   BFA_REQUIRE(workspace_bytes >= need && (need == 0 || workspace),
               "%s: workspace too small (%lld < %lld bytes)", what, (long long)workspace_bytes,
