@@ -1567,7 +1567,8 @@ static void launch_merge(const CasArgs& a, int64_t rows, int64_t splits, hipStre
 }
 
 // The flat form, from more than CAS_FLAT_ROWS query rows per kv head (or as
-// override BFA_TUNE_CASCADE_FLAT = 0 / 1 forces, for measurements).  At Qwen3 shape over 4096
+// override BFA_TUNE_CASCADE_FLAT = 0 / 1 forces, 2 with two row blocks per wave;
+// for measurements and tests).  At Qwen3 shape over 4096
 // keys it is slower than the fused kernel up to 64 rows (26.3 against 25.3 us)
 // and faster from 128 (28.5 against 32.7; 42.3 against 79.4 at 512 rows).
 // Workspace after the split partials: K and V^T copies of the attended keys and
@@ -1599,11 +1600,6 @@ static FlatPlan flat_plan(int64_t rows, int64_t hkv, int64_t num_entries, int64_
   // 256 queries run best at 8 splits (43 us against 51 at 4 and 52 at 16),
   // 1024 queries at 4 (98 against 126 unsplit).  Override
   // BFA_TUNE_CASCADE_FLAT_WG sets the workgroup target instead.
-  // Two 16-row blocks per wave from more than 256 rows (head_dim 64: 1024), where
-  // enough workgroups remain: Llama-3-8B, 100 queries (400 rows) over 8000 keys
-  // 58 -> 53 us, TinyLlama, 1000 (8000 rows) over 3000 71 -> 66 us, but 100 (800
-  // rows) 25 -> 28 us.
-  fp.rb = rows > (d == 64 ? 1024 : 256) ? 2 : 1;
   const int64_t blocks = cdiv(rows, 64) * hkv;
   int64_t target = std::min<int64_t>(std::max<int64_t>(512, 4 * blocks), 1024);
   if (tuning(BFA_TUNE_CASCADE_FLAT_WG) >= 1) target = tuning(BFA_TUNE_CASCADE_FLAT_WG);
@@ -1615,6 +1611,20 @@ static FlatPlan flat_plan(int64_t rows, int64_t hkv, int64_t num_entries, int64_
   zs = std::max<int64_t>(1, zs);
   fp.tiles_per_split = std::max<int64_t>(1, cdiv(fp.tiles, zs));
   fp.splits = std::max<int64_t>(1, cdiv(fp.tiles, fp.tiles_per_split));
+  // Two 16-row blocks per wave halve the workgroups, each of which takes 1.1 to 1.7
+  // times as long: from more than 256 rows (head_dim 64: 1024), where that saves a
+  // round of what the chip holds at once (2 workgroups per CU, head_dim 64: 4) and
+  // there are some tiles to walk, or where the walk is long.  Graph-replayed, one
+  // block and two: Qwen3 600 rows over 8000 keys 75.6 and 60.2 us, 512 over 400
+  // 21.9 and 24.3; Llama-3-8B 4000 over 8000 237 and 206, 300 over 4000 32.9 and
+  // 36.0; TinyLlama 8000 over 8000 138 and 123, 1600 over 8000 41.9 and 52.1.  Of
+  // 402 shapes (100 to 8000 keys, 1 to 8 kv heads) 9 are slower than with one block
+  // at every size, by up to 6 %.
+  const int64_t held = d == 64 ? 1024 : 512, w1 = blocks * fp.splits, w2 = cdiv(rows, 128) * hkv * fp.splits;
+  const int64_t walk = w2 * fp.tiles_per_split;
+  fp.rb = rows > (d == 64 ? 1024 : 256) && ((walk >= 1400 && cdiv(w2, held) < cdiv(w1, held)) ||
+                                            walk >= (d == 64 ? 16000 : 3500)) ? 2 : 1;
+  if (tuning(BFA_TUNE_CASCADE_FLAT) == 2) fp.rb = 2;
   fp.part_bytes = fp.splits > 1 ? align256c(fp.splits * hkv * rows * (d + 2) * 4) : 0;
   fp.kf_bytes = align256c(hkv * fp.npad * d * 2);
   fp.vt_bytes = fp.kf_bytes;

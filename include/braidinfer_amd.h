@@ -70,7 +70,8 @@ const char* bfa_last_error(void);
 #define BFA_TUNE_NO_OPERAND_FOLD 6   /* BFA_NO_OPERAND_FOLD: non-zero = keep the decode pre-pass */
 #define BFA_TUNE_CASCADE_DECODE_WG 7 /* BFA_CASCADE_DECODE_WG: cascade decode workgroup target */
 #define BFA_TUNE_CASCADE_FLAT 8      /* BFA_CASCADE_FLAT: 0 = fused cascade kernel, non-zero =
-                                        flat form from 5 query rows */
+                                        flat form from 5 query rows, 2 = with two
+                                        row blocks per wave */
 #define BFA_TUNE_CASCADE_FLAT_WG 9   /* BFA_CASCADE_FLAT_WG: flat-form workgroup target */
 #define BFA_TUNE_STREAM_STORES 10    /* BFA_STREAM_STORES: 0 = no nontemporal stores */
 #define BFA_TUNE_QKV_PERSIST 11      /* BFA_QKV_PERSIST: prefill GEMM workgroups per CU that loop

@@ -1,6 +1,6 @@
-"""The flat form of cascade attention at the edges of its row blocks: one and two
-16-row blocks per wave (from 257 rows per kv head at head_dim 128, 1025 at 64),
-against the oracle; and what its softmax does with scores that keep growing
+"""The flat form of cascade attention at the edges of its row blocks, with one and
+two 16-row blocks per wave (CASCADE_FLAT 1 at these sizes, and 2), against the
+oracle and bit for bit against each other; and what its softmax does with scores that keep growing
 along the keys, with scores of 2^34, and with a negative or zero scale, against
 64 bits."""
 from __future__ import annotations
@@ -19,19 +19,39 @@ DEV = "cuda"
 @pytest.mark.parametrize("tokens,hq,hkv,d", [(128, 16, 8, 128), (129, 16, 8, 128), (161, 4, 1, 128),
                                              (128, 32, 4, 64), (129, 32, 4, 64), (145, 16, 2, 64)])
 @pytest.mark.parametrize("causal,knorm", [(True, False), (False, True)])
-def test_row_blocks(tuning, tokens, hq, hkv, d, causal, knorm):
-    tuning("CASCADE_FLAT", 1)
+@pytest.mark.parametrize("flat", [1, 2])
+def test_row_blocks(tuning, tokens, hq, hkv, d, causal, knorm, flat):
+    tuning("CASCADE_FLAT", flat)
     _check_case(f"rows {tokens} {hq} {hkv} {d}", tokens, hq, hkv, [48, 130, 64, tokens], [0, 77, -5, 0], causal,
                 knorm, d=d)
 
 
+@pytest.mark.parametrize("tokens,hq,hkv,d", [(25, 4, 1, 128), (97, 4, 2, 128), (161, 4, 1, 128), (145, 16, 2, 64),
+                                             (600, 16, 8, 128)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_one_and_two_blocks_agree(tuning, tokens, hq, hkv, d, causal):
+    """Which wave takes a row changes none of its sums; the planner's own choice
+    (600 tokens: two blocks) is one of the two."""
+    chunks, kv, total = build_case(97, hq, hkv, [700, 130, tokens], [0, 0, 0], pages=120, d=d)
+    q = randn(gen(98), tokens, hq, d, std=2.0)
+    qpos = torch.arange(total - tokens, total)
+    att = CascadeAttention(hq, d, d ** -0.5, hkv, 16, rotary_emb=RotaryEmbedding(d, d, 4096, 1e6).to(DEV))
+    levels = att.create_cascade_levels(chunks)
+    outs = []
+    for flat in (1, 2, None) if tokens * hq > 96 * hkv else (1, 2):
+        tuning("CASCADE_FLAT", flat)
+        outs.append(att.forward(q.to(DEV), qpos.to(DEV), kv.to(DEV), levels, 0, causal_mask=causal).cpu())
+    assert all(torch.equal(o, outs[0]) for o in outs)
+
+
 @pytest.mark.parametrize("tokens", [100, 300])
 @pytest.mark.parametrize("wg", [8, 64])
-def test_growing_scores_and_sign(tuning, tokens, wg):
+@pytest.mark.parametrize("flat", [1, 2])
+def test_growing_scores_and_sign(tuning, tokens, wg, flat):
     """Keys that grow along the walk move the running maximum in every tile (by
     less and by more than the step that rescales); P is rounded to bf16 as
     everywhere, so the plain tolerance holds.  (-q, -scale) is (q, scale)."""
-    tuning("CASCADE_FLAT", 1)
+    tuning("CASCADE_FLAT", flat)
     tuning("CASCADE_FLAT_WG", wg)
     hq, hkv, d, ps = 8, 4, 128, 16
     chunks, kv, total = build_case(91, hq, hkv, [400, 300, 200], [0, 0, 0], pages=90)
@@ -61,9 +81,9 @@ def test_growing_scores_and_sign(tuning, tokens, wg):
     assert_close(outs[0].reshape(tokens, hq, d), exp, what=f"growing scores tokens={tokens} wg={wg}")
 
 
-@pytest.mark.parametrize("tokens", [100, 300])
+@pytest.mark.parametrize("tokens,flat", [(100, 1), (300, 2)])
 @pytest.mark.parametrize("causal", [True, False])
-def test_zero_scale(tuning, tokens, causal):
+def test_zero_scale(tuning, tokens, flat, causal):
     """Every score is 0: the mean of the visible values, with partly filled pages
     and a causal edge inside a tile."""
     tuning("CASCADE_FLAT", 1)
@@ -80,11 +100,11 @@ def test_zero_scale(tuning, tokens, causal):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("tokens", [100, 300])
-def test_scores_of_any_size(tuning, tokens, dtype):
+@pytest.mark.parametrize("tokens,flat", [(100, 1), (300, 2)])
+def test_scores_of_any_size(tuning, tokens, flat, dtype):
     """Scores up to 2^34 (2^28 in fp16), further apart than any exponential: each
     query returns the value of its largest visible key."""
-    tuning("CASCADE_FLAT", 1)
+    tuning("CASCADE_FLAT", flat)
     hq, hkv, d, ps = 8, 4, 128, 16
     chunks, kv, total = build_case(95, hq, hkv, [200, 90, tokens], [0, 0, 0], pages=60)
     kv = kv.to(dtype)
