@@ -40,76 +40,178 @@ __device__ __forceinline__ int64_t lin_weight_row(const LinArgs& q, int64_t n0, 
   }
 }
 
-// Eight neighbouring outputs (columns c .. c + 7) of one token.  SAME: proj_dt,
-// out_dt and res_dt are DT, mid_dt DT or fp32, vec rows and n a multiple
-// of 8; otherwise the dtypes and bounds are the call's.
-template <int DT, bool SAME, bool SWIGLU>
+// Eight neighbouring outputs (columns c .. c + 7) of one token, where proj_dt,
+// out_dt and res_dt are DT, mid_dt DT or fp32, the rows vec and n a multiple of 8.
+template <int DT, bool SWIGLU>
 __device__ __forceinline__ void lin_out8(const LinArgs& q, int64_t row, int64_t c, const float (&a)[8],
                                          const float (&u)[8], const uint4& res) {
   using E = Elem<DT>;
   if (c >= q.n) return;
+  const uint32_t rw[4] = {res.x, res.y, res.z, res.w};
   float y[8];
-  if constexpr (SAME) {
-    const uint32_t rw[4] = {res.x, res.y, res.z, res.w};
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      if constexpr (SWIGLU) {
-        y[t] = E::round(silu_fast(E::round(a[t]))) * E::round(u[t]);
-      } else {
-        float v = a[t];
-        if (q.bias) v = v + load_any(q.bias, q.bias_dt, c + t);
-        v = E::round(v);
-        if (q.res) v = v + E::to_f32(static_cast<uint16_t>((t & 1) ? rw[t >> 1] >> 16 : rw[t >> 1] & 0xffffu));
-        y[t] = v;
-      }
-    }
-    store8<DT>(static_cast<uint16_t*>(q.out) + row * q.ldo + c, y);
-  } else {
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      if constexpr (SWIGLU) {
-        y[t] = round_to(silu_fast(round_to(a[t], q.proj_dt)), q.proj_dt) * round_to(u[t], q.proj_dt);
-      } else {
-        const int64_t cc = min(c + t, q.n - 1);
-        float v = a[t];
-        if (q.bias) v = v + load_any(q.bias, q.bias_dt, cc);
-        v = round_to(v, q.proj_dt);
-        v = v + (q.res ? load_any(q.res, q.res_dt, row * q.ldr + cc) : 0.f);
-        y[t] = round_to(v, q.mid_dt);
-      }
-    }
-    if (q.vec && c + 8 <= q.n) {
-      if (q.out_dt == BFA_DTYPE_BF16) store8<BFA_DTYPE_BF16>(static_cast<uint16_t*>(q.out) + row * q.ldo + c, y);
-      else if (q.out_dt == BFA_DTYPE_F16) store8<BFA_DTYPE_F16>(static_cast<uint16_t*>(q.out) + row * q.ldo + c, y);
-      else store8<BFA_DTYPE_F32>(static_cast<float*>(q.out) + row * q.ldo + c, y);
+  for (int t = 0; t < 8; ++t) {
+    if constexpr (SWIGLU) {
+      y[t] = E::round(silu_fast(E::round(a[t]))) * E::round(u[t]);
     } else {
-#pragma unroll
-      for (int t = 0; t < 8; ++t)
-        if (c + t < q.n) store_any(q.out, q.out_dt, row * q.ldo + c + t, y[t]);
+      float v = a[t];
+      if (q.bias) v = v + load_any(q.bias, q.bias_dt, c + t);
+      v = E::round(v);
+      if (q.res) v = v + E::to_f32(static_cast<uint16_t>((t & 1) ? rw[t >> 1] >> 16 : rw[t >> 1] & 0xffffu));
+      y[t] = v;
     }
   }
+  store8<DT>(static_cast<uint16_t*>(q.out) + row * q.ldo + c, y);
 }
 
 // One token's 16 projection values of a lane; c0 its first output column.
-template <int DT, bool SAME, bool SWIGLU>
+template <int DT, bool SWIGLU>
 __device__ __forceinline__ void lin_finish(const LinArgs& q, int64_t row, int64_t c0, const gemm_f32x4_t (&acc)[4],
                                            const uint4 (&res)[2]) {
   const float lo[8] = {acc[0][0], acc[0][1], acc[0][2], acc[0][3], acc[1][0], acc[1][1], acc[1][2], acc[1][3]};
   const float hi[8] = {acc[2][0], acc[2][1], acc[2][2], acc[2][3], acc[3][0], acc[3][1], acc[3][2], acc[3][3]};
   if constexpr (SWIGLU) {
-    lin_out8<DT, SAME, true>(q, row, c0, lo, hi, res[0]);
+    lin_out8<DT, true>(q, row, c0, lo, hi, res[0]);
   } else {
-    lin_out8<DT, SAME, false>(q, row, c0, lo, lo, res[0]);
-    lin_out8<DT, SAME, false>(q, row, c0 + 8, hi, hi, res[1]);
+    lin_out8<DT, false>(q, row, c0, lo, lo, res[0]);
+    lin_out8<DT, false>(q, row, c0 + 8, hi, hi, res[1]);
+  }
+}
+
+// The general form (any dtypes, any n and row stride) passes a wave's blocks
+// through the LDS, a few at a time, and walks their rows in a loop.  In registers
+// its code, once per block, outgrew the unroller: the accumulators went to scratch,
+// in the main loop too (3000 tokens, K 2048, n = 8004 951 us, against 147 on the
+// projection GEMM's tiles; 127 like this).  A block is 16 tokens of 16 granules of
+// 4 values, granule G of token r at G ^ r (a lane writes 4 granules of one token):
+// plain, the wave's 64 columns in order; SwiGLU, its 32 gate columns, then its 32
+// up columns.
+template <bool SWIGLU>
+__device__ __forceinline__ void lin_stage(gemm_f32x4_t* block, int lane, const gemm_f32x4_t (&acc)[4]) {
+  const int r = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    block[r * 16 + ((SWIGLU ? (j >> 1) * 8 + 2 * g + (j & 1) : 4 * g + j) ^ r)] = acc[j];
+}
+
+// One output from its sum (SwiGLU: and its up sum), bias and residual.
+template <bool SWIGLU>
+__device__ __forceinline__ float lin_value(const LinArgs& q, float a, float u, float bias, float res) {
+  if constexpr (SWIGLU) {
+    return round_to(silu_fast(round_to(a, q.proj_dt)), q.proj_dt) * round_to(u, q.proj_dt);
+  } else {
+    if (q.bias) a = a + bias;
+    return round_to(round_to(a, q.proj_dt) + res, q.mid_dt);
+  }
+}
+
+// `rows` staged tokens of a wave, the first one row0, its first output column c0.
+// Rows that take 16-byte accesses: eight columns a lane; else one, so that the
+// wave's accesses lie next to each other.  A lane keeps its columns, so it reads the
+// bias once; the residual of the next rows is on its way during these rows' work.
+template <bool SWIGLU>
+__device__ __forceinline__ void lin_rows(const LinArgs& q, int64_t row0, int64_t c0, const gemm_f32x4_t* staged,
+                                         int rows, int lane) {
+  constexpr int COLS = SWIGLU ? 32 : 64;
+  rows = static_cast<int>(min<int64_t>(rows, q.m - row0));
+  if (rows <= 0) return;
+  if (q.vec) {
+    constexpr int G8 = COLS / 8, STEP = 64 / G8;
+    const int g = 2 * (lane % G8);
+    const int64_t c = c0 + 4 * g;
+    if (c >= q.n) return;
+    const bool whole = c + 8 <= q.n;
+    float bias[8] = {};
+    if (!SWIGLU && q.bias) {
+#pragma unroll
+      for (int v = 0; v < 8; ++v) bias[v] = load_any(q.bias, q.bias_dt, min(c + v, q.n - 1));
+    }
+    struct Res {
+      uint4 lo, hi;  // 16-bit: lo alone
+    };
+    auto load_res = [&](int t) {
+      Res d{};
+      if (!SWIGLU && q.res && whole) {
+        const char* p = static_cast<const char*>(q.res);
+        const int64_t e = (row0 + min(t, rows - 1)) * q.ldr + c;
+        d.lo = *reinterpret_cast<const uint4*>(p + e * (q.res_dt == BFA_DTYPE_F32 ? 4 : 2));
+        if (q.res_dt == BFA_DTYPE_F32) d.hi = *reinterpret_cast<const uint4*>(p + e * 4 + 16);
+      }
+      return d;
+    };
+    Res cur = load_res(lane / G8);
+    for (int t = lane / G8; t < rows; t += STEP) {
+      const Res next = load_res(t + STEP);
+      const int r = t & 15;
+      const int64_t row = row0 + t;
+      const gemm_f32x4_t* s = staged + t * 16;
+      const gemm_f32x4_t a0 = s[g ^ r], a1 = s[(g + 1) ^ r];
+      const gemm_f32x4_t u0 = SWIGLU ? s[(8 + g) ^ r] : a0, u1 = SWIGLU ? s[(9 + g) ^ r] : a1;
+      const uint32_t w[8] = {cur.lo.x, cur.lo.y, cur.lo.z, cur.lo.w, cur.hi.x, cur.hi.y, cur.hi.z, cur.hi.w};
+      float y[8];
+#pragma unroll
+      for (int v = 0; v < 8; ++v) {
+        float res = 0.f;
+        if (!SWIGLU && q.res) {
+          const uint32_t h = (v & 1) ? w[v >> 1] >> 16 : w[v >> 1] & 0xffffu;
+          if (!whole) res = load_any(q.res, q.res_dt, row * q.ldr + min(c + v, q.n - 1));
+          else if (q.res_dt == BFA_DTYPE_F32) res = __uint_as_float(w[v]);
+          else res = q.res_dt == BFA_DTYPE_BF16 ? bf16_bits_to_f32(h) : f16_bits_to_f32(h);
+        }
+        y[v] = lin_value<SWIGLU>(q, v < 4 ? a0[v & 3] : a1[v & 3], v < 4 ? u0[v & 3] : u1[v & 3], bias[v], res);
+      }
+      cur = next;
+      if (whole) {
+        if (q.out_dt == BFA_DTYPE_BF16) store8<BFA_DTYPE_BF16>(static_cast<uint16_t*>(q.out) + row * q.ldo + c, y);
+        else if (q.out_dt == BFA_DTYPE_F16) store8<BFA_DTYPE_F16>(static_cast<uint16_t*>(q.out) + row * q.ldo + c, y);
+        else store8<BFA_DTYPE_F32>(static_cast<float*>(q.out) + row * q.ldo + c, y);
+      } else {
+#pragma unroll
+        for (int v = 0; v < 8; ++v)
+          if (c + v < q.n) store_any(q.out, q.out_dt, row * q.ldo + c + v, y[v]);
+      }
+    }
+    return;
+  }
+  constexpr int STEP = 64 / COLS, U = 8;  // rows at a time
+  const float* f = reinterpret_cast<const float*>(staged);
+  const int col = lane % COLS;
+  const int64_t c = c0 + col;
+  if (c >= q.n) return;
+  const float bias = !SWIGLU && q.bias ? load_any(q.bias, q.bias_dt, c) : 0.f;
+  struct Res {
+    uint32_t v[U];
+  };
+  auto load_res = [&](int t) {
+    Res d{};
+    if (!SWIGLU && q.res) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) d.v[u] = ld_word(q.res, q.res_dt, (row0 + min(t + u * STEP, rows - 1)) * q.ldr + c);
+    }
+    return d;
+  };
+  Res cur = load_res(lane / COLS);
+  for (int t0 = lane / COLS; t0 < rows; t0 += U * STEP) {
+    const Res next = load_res(t0 + U * STEP);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int t = t0 + u * STEP;
+      if (t >= rows) break;
+      const int r = t & 15, o = t * 64 + (col & 3);
+      const float a = f[o + 4 * ((col >> 2) ^ r)], up = SWIGLU ? f[o + 4 * ((8 + (col >> 2)) ^ r)] : a;
+      const float res = !SWIGLU && q.res ? word_value(cur.v[u], q.res_dt, q.res, (row0 + t) * q.ldr + c) : 0.f;
+      store_any(q.out, q.out_dt, (row0 + t) * q.ldo + c, lin_value<SWIGLU>(q, a, up, bias, res));
+    }
+    cur = next;
   }
 }
 
 // The lane's residual elements, ahead of their use (columns past n are clamped;
 // their results are not stored).
-template <bool SAME, bool SWIGLU>
+template <bool SWIGLU>
 __device__ __forceinline__ void lin_residual(const LinArgs& q, int64_t row, int64_t c0, uint4 (&res)[2]) {
   res[0] = res[1] = make_uint4(0, 0, 0, 0);
-  if constexpr (SAME && !SWIGLU) {
+  if constexpr (!SWIGLU) {
     if (q.res) {
 #pragma unroll
       for (int h = 0; h < 2; ++h)
@@ -150,6 +252,21 @@ __global__ __launch_bounds__(RW * CW * 64, 2) void linear_gemm_kernel(LinArgs q)
                            static_cast<int>(cdiv(q.m - wm0, 16)), acc);
     return;
   }
+  if constexpr (!SAME) {
+    constexpr int HB = T::LDS_U4 / (T::NW * 256) < MA ? T::LDS_U4 / (T::NW * 256) : MA;  // blocks of 4 KiB at a time
+    static_assert(HB >= 1, "a block per wave takes the ring's place");
+    gemm_f32x4_t* staged = reinterpret_cast<gemm_f32x4_t*>(lds) + wid * (HB * 256);
+    __syncthreads();  // the ring's last reads are done
+#pragma unroll
+    for (int h = 0; h < MA; h += HB) {
+#pragma unroll
+      for (int i = 0; i < HB && h + i < MA; ++i) lin_stage<SWIGLU>(staged + i * 256, lane, acc[h + i]);
+      asm volatile("" ::: "memory");  // the wave's own LDS writes precede its reads, and these the next writes
+      lin_rows<SWIGLU>(q, wm0 + h * 16, n0 + wc * (SWIGLU ? 32 : 64), staged, min(HB, MA - h) * 16, lane);
+      asm volatile("" ::: "memory");
+    }
+    return;
+  }
   const int64_t c0 = n0 + (SWIGLU ? wc * 32 + (lane >> 4) * 8 : wc * 64 + (lane >> 4) * 16);
   const int64_t r0 = wm0 + (lane & 15);
   // the residual rows of half the blocks are requested together (of all of
@@ -159,10 +276,10 @@ __global__ __launch_bounds__(RW * CW * 64, 2) void linear_gemm_kernel(LinArgs q)
   for (int h = 0; h < MA; h += H) {
     uint4 res[H][2];
 #pragma unroll
-    for (int i = 0; i < H; ++i) lin_residual<SAME, SWIGLU>(q, min(r0 + (h + i) * 16, q.m - 1), c0, res[i]);
+    for (int i = 0; i < H; ++i) lin_residual<SWIGLU>(q, min(r0 + (h + i) * 16, q.m - 1), c0, res[i]);
 #pragma unroll
     for (int i = 0; i < H && h + i < MA; ++i)
-      if (r0 + (h + i) * 16 < q.m) lin_finish<DT, SAME, SWIGLU>(q, r0 + (h + i) * 16, c0, acc[h + i], res[i]);
+      if (r0 + (h + i) * 16 < q.m) lin_finish<DT, SWIGLU>(q, r0 + (h + i) * 16, c0, acc[h + i], res[i]);
   }
 }
 
@@ -178,15 +295,23 @@ __global__ __launch_bounds__(256) void linear_reduce_kernel(LinArgs q, int ma, i
   gemm_tile(q.tiles_m, q.tiles_n, q.full + rest, tm, tn);
   const int64_t row0 = (static_cast<int64_t>(tm) * rw * ma + wr * ma + i) * 16, row = row0 + (lane & 15);
   if (row0 >= q.m) return;  // no partials there
-  const int64_t c0 = SWIGLU ? (static_cast<int64_t>(tn) * cw + wc) * 32 + (lane >> 4) * 8
-                            : (static_cast<int64_t>(tn) * cw + wc) * 64 + (lane >> 4) * 16;
+  const int64_t w0 = (static_cast<int64_t>(tn) * cw + wc) * (SWIGLU ? 32 : 64);  // the wave's first output column
+  const int64_t c0 = w0 + (lane >> 4) * (SWIGLU ? 8 : 16);
   uint4 res[2];
-  lin_residual<SAME, SWIGLU>(q, min(row, q.m - 1), c0, res);
+  if constexpr (SAME) lin_residual<SWIGLU>(q, min(row, q.m - 1), c0, res);
   gemm_f32x4_t acc[4];
   const int64_t stride = static_cast<int64_t>(per) * 256;
   gemm_sum_part(reinterpret_cast<const gemm_f32x4_t*>(q.part) + (static_cast<int64_t>(rest) * q.splits * per + in) * 256 + lane,
                 stride, q.splits, acc);
-  if (row < q.m) lin_finish<DT, SAME, SWIGLU>(q, row, c0, acc, res);
+  if constexpr (SAME) {
+    if (row < q.m) lin_finish<DT, SWIGLU>(q, row, c0, acc, res);
+  } else {
+    __shared__ gemm_f32x4_t blocks[4][256];
+    gemm_f32x4_t* staged = blocks[threadIdx.x >> 6];
+    lin_stage<SWIGLU>(staged, lane, acc);
+    asm volatile("" ::: "memory");  // the wave's own LDS writes precede its reads
+    lin_rows<SWIGLU>(q, row0, w0, staged, 16, lane);
+  }
 }
 
 // ------------------------------------------------------------------- host

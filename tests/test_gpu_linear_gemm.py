@@ -58,6 +58,35 @@ def test_general_forms(tuning, splits):
     assert_close(y, (x.float() @ w.float().t() + r.float()).half().to(x.dtype), what="attention output")
 
 
+@pytest.mark.parametrize("tile", range(8))
+@pytest.mark.parametrize("splits", [1, 3])
+def test_general_forms_on_every_tile(tuning, tile, splits):
+    """The general epilogue, one token past a tile: rows that do not take 16-byte
+    stores (n odd, and a multiple of 4) with a bias or an fp32 residual, SwiGLU of
+    an odd width, and the attention output's fp16 sum on rows that do."""
+    tuning("GEMM_TILE", tile)
+    tuning("GEMM_SPLITS", splits)
+    g = gen(4300 + tile)
+    t, k = TILE_TOKENS[tile] + 1, 192
+    x = randn(g, t, k)
+    for n in (299, 300):
+        w, b = randn(g, n, k, std=0.03), torch.randn(n, generator=g)
+        assert_close(linear(x.to(DEV), w.to(DEV), b.to(DEV)), R.linear(x, w, b), what=f"bias n={n} tile={tile}")
+        r = torch.randn(t, n, generator=g)
+        assert_close(linear_add_residual(x.to(DEV), w.to(DEV), r.to(DEV)),
+                     (R.linear(x, w).float() + r).to(x.dtype), what=f"fp32 residual n={n} tile={tile}",
+                     # one bf16 ulp of the projection: its rounding precedes the addition
+                     slack=2.0 ** -7 * R.linear(x, w).float().abs(), max_slack_frac=1e-3)
+    w2 = randn(g, 2 * 203, k, std=0.05)
+    exp = R.gate_up_silu_and_mul(x, w2)
+    # silu and up are rounded before their product: two more ulps at most
+    assert_close(gate_up_silu_and_mul(x.to(DEV), w2.to(DEV)), exp, what=f"gate_up tile={tile}",
+                 slack=2.0 ** -6 * exp.float().abs(), max_slack_frac=1e-4)
+    w, r = randn(g, 328, k, std=0.03), randn(g, t, 328)
+    assert_close(attention_output(x.to(DEV), w.to(DEV), r.to(DEV)),
+                 (x.float() @ w.float().t() + r.float()).half().to(x.dtype), what=f"attention output tile={tile}")
+
+
 def test_without_workspace():
     """A caller that brings no workspace gets the unsplit plan: the same result
     up to the order of the fp32 sums, so at most one bf16 rounding apart."""
