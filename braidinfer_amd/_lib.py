@@ -228,31 +228,53 @@ def get_tuning(name: str) -> int | None:
     return _tuning_seen[name]
 
 
-_workspaces: dict = {}
+class Scratch:
+    """A device buffer for the kernels of one call, which holds `lock` from
+    reserve() until its last launch is queued: a call queues several kernels with
+    the GIL released, and another thread's on the same stream must not fall
+    between them."""
+
+    __slots__ = ("lock", "device", "buf", "ptr", "size")
+
+    def __init__(self, device: torch.device):
+        self.lock = threading.RLock()
+        self.device, self.buf, self.ptr, self.size = device, None, 0, 0
+
+    def reserve(self, nbytes: int) -> None:
+        """Makes it at least `nbytes` long (16-byte aligned, never empty); allocates
+        on the current stream."""
+        if self.size < nbytes or self.buf is None:
+            buf = torch.empty(max(nbytes, 16, 2 * self.size), dtype=torch.uint8, device=self.device)
+            self.buf, self.ptr, self.size = buf, buf.data_ptr(), buf.numel()
 
 
-def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
-    """A device scratch buffer of at least `nbytes` (16-byte aligned) for a
-    kernel launched on the current stream.  Outside graph capture one buffer
-    per (device, stream) is kept and reused: launches on one stream are ordered,
-    so a call's kernels finish with it before the next call's start.  Under
-    graph capture a fresh allocation from the graph's pool is returned, so a
-    captured graph never shares (or outlives) the eager buffer."""
-    idx = device.index if device.index is not None else torch.cuda.current_device()
-    stream = stream_of(device)
+_workspaces: dict = {}  # (device index, stream handle) -> Scratch
+
+
+def scratch(device: torch.device) -> Scratch:
+    """The scratch buffer for a call on the current stream; use it as
+
+        ws = scratch(device)
+        with ws.lock:
+            ws.reserve(nbytes)
+            ...launch with ws.ptr, ws.size...
+
+    Outside graph capture one per (device, stream) is kept and reused: launches on
+    one stream are ordered, and the lock keeps one call's together, so a call's
+    kernels finish with it before the next call's start.  Under graph capture a
+    fresh one from the graph's pool, so a captured graph never shares (or
+    outlives) the eager buffer."""
     if torch.cuda.is_current_stream_capturing():
-        return torch.empty(max(nbytes, 16), dtype=torch.uint8, device=device)
-    key = (idx, stream)
-    buf = _workspaces.get(key)
-    if buf is None or buf.numel() < nbytes:
-        buf = torch.empty(max(nbytes, 16, 0 if buf is None else 2 * buf.numel()), dtype=torch.uint8,
-                          device=device)
-        _workspaces[key] = buf
-    return buf
+        return Scratch(device)
+    key = (device.index if device.index is not None else torch.cuda.current_device(), stream_of(device))
+    s = _workspaces.get(key)
+    if s is None:
+        s = _workspaces.setdefault(key, Scratch(device))
+    return s
 
 
 def clear_workspaces(device: torch.device | int | None = None) -> int:
-    """Releases the reused scratch buffers of workspace() (all devices, or one)
+    """Releases the reused scratch buffers of scratch() (all devices, or one)
     back to torch's caching allocator and returns the bytes released.  A buffer
     grows to the largest call made on its stream and is otherwise kept for the
     life of the process; call this after a one-off large call (an 8192-token
@@ -264,8 +286,10 @@ def clear_workspaces(device: torch.device | int | None = None) -> int:
         idx = device if isinstance(device, int) else (
             device.index if device.index is not None else torch.cuda.current_device())
     freed = 0
-    for key in [k for k in _workspaces if idx is None or k[0] == idx]:
-        freed += _workspaces.pop(key).numel()
+    for key in [k for k in list(_workspaces) if idx is None or k[0] == idx]:
+        s = _workspaces.pop(key, None)  # (a call that holds it keeps its memory until it has launched)
+        if s is not None:
+            freed += s.size
     return freed
 
 

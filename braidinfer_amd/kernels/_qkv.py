@@ -177,50 +177,28 @@ def fused_rmsnorm_qkv(
             size_fn = ("bfa_fused_rmsnorm_qkv_append_workspace_size" if paged_kv is not None
                        else "bfa_fused_rmsnorm_qkv_workspace_size")
             ws_bytes = _lib.workspace_size(size_fn, tokens, hidden, qkv_dim, hd)
-            workspace = _lib.workspace(dev, ws_bytes)
             no_cache = (None, 0, 0, 0, 0, 0, 0, 0, None, 0, 0, None, None, 0, 0, None, 0, 0, 0)
-            rc = _FOLDED()(
-                input.data_ptr(), _lib.dtype_code(input), tokens, hidden, input.stride(0), float(eps),
-                wf.data_ptr(), _lib.dtype_code(wf), qkv_dim, wf.stride(0),
-                _lib.ptr(qkv_bias), _lib.dtype_code(qkv_bias) if qkv_bias is not None else 0,
-                num_q_heads, num_kv_heads, _lib.dtype_code(qkv_dtype),
-                _lib.ptr(positions), _lib.dtype_code(positions) if positions is not None else 0,
-                _lib.ptr(cos_sin_cache), cos_sin_cache.shape[0] if cos_sin_cache is not None else 0,
-                out.data_ptr(), _lib.dtype_code(out), out.stride(0),
-                workspace.data_ptr(), workspace.numel(),
-                *(cache_args if paged_kv is not None else no_cache),
-                _lib.status_word(dev).data_ptr(), _lib.stream_of(dev),
-            )
+            ws = _lib.scratch(dev)
+            with ws.lock:
+                ws.reserve(ws_bytes)
+                rc = _FOLDED()(
+                    input.data_ptr(), _lib.dtype_code(input), tokens, hidden, input.stride(0), float(eps),
+                    wf.data_ptr(), _lib.dtype_code(wf), qkv_dim, wf.stride(0),
+                    _lib.ptr(qkv_bias), _lib.dtype_code(qkv_bias) if qkv_bias is not None else 0,
+                    num_q_heads, num_kv_heads, _lib.dtype_code(qkv_dtype),
+                    _lib.ptr(positions), _lib.dtype_code(positions) if positions is not None else 0,
+                    _lib.ptr(cos_sin_cache), cos_sin_cache.shape[0] if cos_sin_cache is not None else 0,
+                    out.data_ptr(), _lib.dtype_code(out), out.stride(0), ws.ptr, ws.size,
+                    *(cache_args if paged_kv is not None else no_cache),
+                    _lib.status_word(dev).data_ptr(), _lib.stream_of(dev),
+                )
             if rc == 0:
                 return out
             if rc != _ERR_UNSUPPORTED:
                 _lib.raise_error(rc)
     if tokens == 0:
         return out
-    if paged_kv is not None:
-        ws_bytes = _lib.workspace_size("bfa_fused_rmsnorm_qkv_append_workspace_size", tokens, hidden,
-                                       qkv_dim, hd)
-        workspace = _lib.workspace(dev, ws_bytes)
-        _lib.call(
-            "bfa_fused_rmsnorm_qkv_append",
-            input.data_ptr(), _lib.dtype_code(input), tokens, hidden, input.stride(0),
-            norm_weight.data_ptr(), _lib.dtype_code(norm_weight), float(eps), int(mixed_rounding),
-            w.data_ptr(), _lib.dtype_code(w), qkv_dim, w.stride(0),
-            _lib.ptr(qkv_bias), _lib.dtype_code(qkv_bias) if qkv_bias is not None else 0,
-            num_q_heads, num_kv_heads, _lib.dtype_code(qkv_dtype),
-            _lib.ptr(q_norm_weight), _lib.ptr(k_norm_weight),
-            _lib.dtype_code(qn_dtype) if qn_dtype is not None else 0, float(qk_norm_eps),
-            _lib.dtype_code(qk_norm_out_dtype or input.dtype),
-            _lib.ptr(positions), _lib.dtype_code(positions) if positions is not None else 0,
-            _lib.ptr(cos_sin_cache), cos_sin_cache.shape[0] if cos_sin_cache is not None else 0,
-            out.data_ptr(), _lib.dtype_code(out), out.stride(0),
-            workspace.data_ptr(), workspace.numel(), *cache_args,
-            _lib.status_word(dev).data_ptr(), _lib.stream_of(dev),
-        )
-        return out
-    ws_bytes = _lib.workspace_size("bfa_fused_rmsnorm_qkv_workspace_size", tokens, hidden, qkv_dim, hd)
-    workspace = _lib.workspace(dev, ws_bytes)
-    rc = _FUSED()(
+    args = (
         input.data_ptr(), _lib.dtype_code(input), tokens, hidden, input.stride(0),
         norm_weight.data_ptr(), _lib.dtype_code(norm_weight), float(eps), int(mixed_rounding),
         w.data_ptr(), _lib.dtype_code(w), qkv_dim, w.stride(0),
@@ -232,9 +210,20 @@ def fused_rmsnorm_qkv(
         _lib.ptr(positions), _lib.dtype_code(positions) if positions is not None else 0,
         _lib.ptr(cos_sin_cache), cos_sin_cache.shape[0] if cos_sin_cache is not None else 0,
         out.data_ptr(), _lib.dtype_code(out), out.stride(0),
-        workspace.data_ptr(), workspace.numel(),
-        _lib.status_word(dev).data_ptr(), _lib.stream_of(dev),
     )
+    ws = _lib.scratch(dev)
+    if paged_kv is not None:
+        ws_bytes = _lib.workspace_size("bfa_fused_rmsnorm_qkv_append_workspace_size", tokens, hidden,
+                                       qkv_dim, hd)
+        with ws.lock:
+            ws.reserve(ws_bytes)
+            _lib.call("bfa_fused_rmsnorm_qkv_append", *args, ws.ptr, ws.size, *cache_args,
+                      _lib.status_word(dev).data_ptr(), _lib.stream_of(dev))
+        return out
+    ws_bytes = _lib.workspace_size("bfa_fused_rmsnorm_qkv_workspace_size", tokens, hidden, qkv_dim, hd)
+    with ws.lock:
+        ws.reserve(ws_bytes)
+        rc = _FUSED()(*args, ws.ptr, ws.size, _lib.status_word(dev).data_ptr(), _lib.stream_of(dev))
     if rc < 0:
         _lib.raise_error(rc)
     return out

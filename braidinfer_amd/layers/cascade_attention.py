@@ -160,18 +160,20 @@ class CascadeAttention:
             qpos = qpos.long()
         ws_bytes = _lib.workspace_size("bfa_cascade_attention_workspace_size", tokens, self.num_heads, hkv, d,
                                        entries, self.page_size)
-        ws = _lib.workspace(dev, ws_bytes)
         st = kv_cache.stride()
-        _lib.call(
-            "bfa_cascade_attention",
-            query.data_ptr(), _lib.dtype_code(query), tokens, self.num_heads,
-            query.stride(0), query.stride(1), qpos.data_ptr(), _lib.dtype_code(qpos),
-            kv_cache.data_ptr(), num_pages, hkv, self.page_size, d, st[0], st[1], st[2], st[3],
-            entries, _lib.ptr(e_page), _lib.ptr(e_kstart), _lib.ptr(e_delta), _lib.ptr(e_info),
-            _lib.ptr(cs), max_pos, _lib.ptr(kn_w), kn_dt, kn_eps,
-            float(self.scale), int(bool(causal_mask)), out.data_ptr(), hd,
-            ws.data_ptr(), ws.numel(), _lib.status_word(dev).data_ptr(), _lib.stream_of(dev),
-        )
+        ws = _lib.scratch(dev)
+        with ws.lock:
+            ws.reserve(ws_bytes)
+            _lib.call(
+                "bfa_cascade_attention",
+                query.data_ptr(), _lib.dtype_code(query), tokens, self.num_heads,
+                query.stride(0), query.stride(1), qpos.data_ptr(), _lib.dtype_code(qpos),
+                kv_cache.data_ptr(), num_pages, hkv, self.page_size, d, st[0], st[1], st[2], st[3],
+                entries, _lib.ptr(e_page), _lib.ptr(e_kstart), _lib.ptr(e_delta), _lib.ptr(e_info),
+                _lib.ptr(cs), max_pos, _lib.ptr(kn_w), kn_dt, kn_eps,
+                float(self.scale), int(bool(causal_mask)), out.data_ptr(), hd,
+                ws.ptr, ws.size, _lib.status_word(dev).data_ptr(), _lib.stream_of(dev),
+            )
         return out
 
     __call__ = forward

@@ -68,16 +68,20 @@ def _run(x: torch.Tensor, weight: torch.Tensor, n: int, mode: int, bias=None, re
             raise ValueError(f"bias has {bias.numel()} elements, the layer has {n} outputs")
         bias = bias.detach().contiguous()
     ws_bytes = _lib.workspace_size("bfa_linear_workspace_size", tokens, k, n, mode)
-    ws = _lib.workspace(dev, ws_bytes) if ws_bytes else None
     code = _lib.dtype_code(x2)
-    _lib.call(
-        "bfa_linear", x2.data_ptr(), code, tokens, k, x2.stride(0),
-        weight.data_ptr(), n, weight.stride(0), _lib.ptr(bias),
-        _lib.dtype_code(bias) if bias is not None else 0, mode,
-        code if proj_dtype is None else proj_dtype,
-        _lib.ptr(r2), _lib.dtype_code(r2) if r2 is not None else 0, r2.stride(0) if r2 is not None else n,
-        sum_dtype, out.data_ptr(), code if out_t == x2.dtype else _lib.dtype_code(out), n,
-        None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _lib.stream_of(dev))
+    args = (x2.data_ptr(), code, tokens, k, x2.stride(0),
+            weight.data_ptr(), n, weight.stride(0), _lib.ptr(bias),
+            _lib.dtype_code(bias) if bias is not None else 0, mode,
+            code if proj_dtype is None else proj_dtype,
+            _lib.ptr(r2), _lib.dtype_code(r2) if r2 is not None else 0, r2.stride(0) if r2 is not None else n,
+            sum_dtype, out.data_ptr(), code if out_t == x2.dtype else _lib.dtype_code(out), n)
+    if ws_bytes:
+        ws = _lib.scratch(dev)
+        with ws.lock:
+            ws.reserve(ws_bytes)
+            _lib.call("bfa_linear", *args, ws.ptr, ws.size, _lib.stream_of(dev))
+    else:
+        _lib.call("bfa_linear", *args, None, 0, _lib.stream_of(dev))
     return out if x.dim() == 2 else out.view(*x.shape[:-1], n)
 
 
