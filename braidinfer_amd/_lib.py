@@ -12,6 +12,7 @@ from __future__ import annotations
 import ctypes
 import importlib.machinery
 import importlib.util
+import sysconfig
 import threading
 import warnings
 from ctypes import c_float, c_int, c_int64, c_void_p
@@ -151,20 +152,22 @@ def exported_symbols():
     return list(_SIGNATURES)
 
 
-_entries = None  # the module of vector-call entry points (csrc/pyentry.cpp)
+# The vector-call entry points (csrc/pyentry.cpp), by the ABI tag of the interpreter
+# that built them: another interpreter does not find them, and calls the library
+# through ctypes.
+ENTRY_PATH = LIB_PATH.parent / ("_bfa_entry" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
+_entries = None  # that module, or load()
 
 
 def _load_entries():
     global _entries
-    load()  # the library first: one copy serves both, and its absence is reported there
+    lib = load()  # the library first: one copy serves both, and its absence is reported there
     with _lock:
         if _entries is None:
-            path = LIB_PATH.parent / "_bfa_entry.so"
-            if not path.exists():
-                raise RuntimeError(
-                    f"braidinfer_amd entry module not found at {path}; "
-                    "build it with `python -m braidinfer_amd.build`")
-            loader = importlib.machinery.ExtensionFileLoader("_bfa_entry", str(path))
+            if not ENTRY_PATH.exists():
+                _entries = lib
+                return _entries
+            loader = importlib.machinery.ExtensionFileLoader("_bfa_entry", str(ENTRY_PATH))
             mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_bfa_entry", loader))
             loader.exec_module(mod)
             _entries = mod

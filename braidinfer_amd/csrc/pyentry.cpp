@@ -1,8 +1,9 @@
 // CPython module _bfa_entry: the C ABI's entry points as vector-call functions.
 //
 // Each entry takes the C function's arguments in order: int for int and int64_t,
-// int or None for pointers, a number for float (or a ctypes scalar of these); it
-// returns the C result.  ctypes
+// int or None for pointers, a number for float, and what ctypes takes in their place
+// (its scalars, arrays, pointers and byref(), an object's _as_parameter_); it returns
+// the C result.  An int that the C type does not hold raises OverflowError.  ctypes
 // converts the 50 arguments of a fused call through Python-level argument types in
 // about 5 us, as long as two kernel launches; these functions take 1.
 #define PY_SSIZE_T_CLEAN
@@ -17,18 +18,47 @@
 
 namespace {
 
+// Address that ctypes passes for an array, a pointer, byref() or bytes:
+// ctypes.cast(o, ctypes.c_void_p).value, a new reference; null with a TypeError.
+PyObject* ctypes_address(PyObject* o) {
+  PyObject* address = nullptr;
+  if (PyObject* ctypes = PyUnicode_Check(o) ? nullptr : PyImport_ImportModule("ctypes")) {
+    PyObject* type = PyObject_GetAttrString(ctypes, "c_void_p");
+    PyObject* pointer = type ? PyObject_CallMethod(ctypes, "cast", "OO", o, type) : nullptr;
+    if (pointer) address = PyObject_GetAttrString(pointer, "value");
+    Py_XDECREF(pointer);
+    Py_XDECREF(type);
+    Py_DECREF(ctypes);
+  }
+  if (!address) {
+    PyErr_Clear();
+    PyErr_Format(PyExc_TypeError, "an int, None or a ctypes object is required for a pointer, not %s",
+                 Py_TYPE(o)->tp_name);
+  }
+  return address;
+}
+
 template <class T>
 bool from_py(PyObject* o, T& v) {
   if (!PyLong_Check(o) && !PyFloat_Check(o) && o != Py_None) {
     // a ctypes scalar (c_void_p, c_float, ...) stands for its value
-    if (PyObject* value = PyObject_GetAttrString(o, "value")) {
+    for (const char* name : {"value", "_as_parameter_"}) {
+      PyObject* value = PyObject_GetAttrString(o, name);
+      if (!value) {
+        PyErr_Clear();
+        continue;
+      }
       const bool plain = PyLong_Check(value) || PyFloat_Check(value) || value == Py_None;
       const bool ok = plain && from_py(value, v);
-      if (!plain) PyErr_SetString(PyExc_TypeError, "an int, a float, None or a ctypes scalar is required");
       Py_DECREF(value);
+      if (plain) return ok;
+    }
+    if constexpr (std::is_pointer_v<T>) {
+      PyObject* value = ctypes_address(o);
+      const bool ok = value && from_py(value, v);
+      Py_XDECREF(value);
       return ok;
     }
-    PyErr_Clear();
   }
   if constexpr (std::is_pointer_v<T>) {
     if (o == Py_None) {
