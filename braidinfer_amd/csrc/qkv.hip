@@ -3087,8 +3087,7 @@ extern "C" int bfa_fused_rmsnorm_qkv(const void* x, int x_dtype, int64_t tokens,
 // A kernel that resolved the slots first cost 3.5 us of a 64-token decode call.
 extern "C" int64_t bfa_fused_rmsnorm_qkv_append_workspace_size(int64_t tokens, int64_t hidden,
                                                                int64_t qkv_dim, int64_t head_dim) {
-  if (tokens <= 0) return 0;
-  return bfa_fused_rmsnorm_qkv_workspace_size(tokens, hidden, qkv_dim, head_dim) + align256(tokens * 8);
+  return bfa_fused_rmsnorm_qkv_workspace_size(tokens, hidden, qkv_dim, head_dim);
 }
 
 // The cache arguments of the fused append, checked and gathered into `a`.
@@ -3137,7 +3136,7 @@ extern "C" int bfa_fused_rmsnorm_qkv_append(
   const int64_t heads = num_q_heads + 2 * num_kv_heads;
   BFA_REQUIRE(heads > 0 && qkv_dim % heads == 0, "%s: bad head geometry", what);
   const QkvPlan p = make_plan(tokens, qkv_dim, hidden, qkv_dim / heads);
-  const int64_t need = p.operand_bytes + p.need_bytes + align256(tokens * 8);  // (the size this entry has always asked for)
+  const int64_t need = p.operand_bytes + p.need_bytes;
   BFA_REQUIRE(workspace && aligned16(workspace) && workspace_bytes >= need,
               "%s: workspace too small (%lld < %lld bytes)", what, (long long)workspace_bytes, (long long)need);
   const CacheEpi ce{layer_cache, cache_dtype, stride_kv, stride_head, write_kv_out ? 0 : 1, &a};
@@ -3190,7 +3189,7 @@ extern "C" int bfa_fused_rmsnorm_qkv_folded(
     return set_error(BFA_ERR_UNSUPPORTED,
                      "%s: the prefill epilogue (more than 64 tokens, head_dim 32, 64 or 128) or the "
                      "column-pair decode shapes (17-64 bf16 tokens) only", what);
-  const int64_t need = p.operand_bytes + p.need_bytes + (layer_cache && p.decode ? align256(tokens * 8) : 0);
+  const int64_t need = p.operand_bytes + p.need_bytes;
   BFA_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace),
               "%s: workspace too small (%lld < %lld bytes)", what, (long long)workspace_bytes, (long long)need);
   char* ws = static_cast<char*>(workspace);

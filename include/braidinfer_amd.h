@@ -285,8 +285,7 @@ int bfa_fused_rmsnorm_qkv_noalloc(const void* x, int x_dtype, int64_t tokens, in
  * the kernel's own Gram diagonal), x in W's dtype; other shapes return
  * BFA_ERR_UNSUPPORTED before any launch.  Against the oracle the bf16 rounding
  * moves from the operand to the weight, within the same tolerance.
- * workspace: bfa_fused_rmsnorm_qkv_workspace_size() bytes, and with an append at
- * decode counts bfa_fused_rmsnorm_qkv_append_workspace_size(). */
+ * workspace: bfa_fused_rmsnorm_qkv_workspace_size() bytes, with an append too. */
 int bfa_fold_rmsnorm_weight(const void* qkv_weight, int w_dtype, int64_t qkv_dim, int64_t hidden,
                             int64_t w_stride, const void* norm_weight, int nw_dtype, void* folded,
                             int64_t folded_stride, void* stream);
@@ -375,8 +374,8 @@ int bfa_append_paged_kv(const void* k, const void* v, int kv_dtype, int64_t num_
  * positions in their sequences, which may differ from the RoPE positions).
  * write_kv_out = 0 leaves the k/v columns of out unwritten (q only).  Cache
  * strides must be multiples of 4 elements and the cache 16-byte aligned.
- * workspace: bfa_fused_rmsnorm_qkv_append_workspace_size() bytes (the fused
- * workspace plus tokens x 8 bytes). */
+ * workspace: bfa_fused_rmsnorm_qkv_append_workspace_size() bytes, the size of
+ * bfa_fused_rmsnorm_qkv's. */
 int64_t bfa_fused_rmsnorm_qkv_append_workspace_size(int64_t tokens, int64_t hidden,
                                                     int64_t qkv_dim, int64_t head_dim);
 int bfa_fused_rmsnorm_qkv_append(

@@ -52,6 +52,11 @@ def test_workspace_size_plan():
     assert ws == 8192 * 4096 * 2
     ws = _lib.call("bfa_fused_rmsnorm_qkv_workspace_size", 300, 512, 800, 80)
     assert ws == (300 * 512 * 2 + 255) // 256 * 256 + (300 * 800 * 4 + 255) // 256 * 256
+    # the append needs nothing more: the epilogues find the cache slots themselves
+    for shape in ((0, 4096, 6144, 128), (5, 2048, 2560, 64), (64, 4096, 6144, 128), (700, 1024, 4096, 128),
+                  (300, 512, 800, 80)):
+        assert (_lib.call("bfa_fused_rmsnorm_qkv_append_workspace_size", *shape)
+                == _lib.call("bfa_fused_rmsnorm_qkv_workspace_size", *shape))
 
 
 def test_cascade_workspace_size_plan(tuning):
