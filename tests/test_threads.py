@@ -1,6 +1,7 @@
-"""Scratch buffers between host threads: a buffer is kept per (device, stream) and
+"""Scratch buffers, between host threads and where memory ends: a buffer is kept per (device, stream) and
 a call queues several kernels over it with the GIL released, so two threads on
-one stream must not interleave theirs.  On the CPU, with entry points that only
+one stream must not interleave theirs; the partial sums of a linear layer above 64
+tokens are optional.  On the CPU, with entry points that only
 record; the GPU counterpart is tests/test_gpu_threads.py."""
 from __future__ import annotations
 
@@ -116,3 +117,20 @@ def test_the_lock_is_given_back_after_an_error(host):
     host(8192, bfa_linear=rec)
     call()
     assert rec.sizes[0] >= 8192
+
+
+@pytest.mark.parametrize("tokens,served", [(300, True), (64, False)])
+def test_linear_without_memory_for_its_partial_sums(host, monkeypatch, tokens, served):
+    def full(self, nbytes):
+        raise torch.cuda.OutOfMemoryError("no memory")
+
+    rec = Recorder(19)
+    host(4096, bfa_linear=rec)
+    monkeypatch.setattr(_lib.Scratch, "reserve", full)
+    x = torch.zeros(300, 64, dtype=torch.bfloat16)
+    if served:
+        linear(x[:tokens], x[:64])
+        assert rec.sizes == [0]
+    else:
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            linear(x[:tokens], x[:64])
