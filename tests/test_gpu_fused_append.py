@@ -113,13 +113,27 @@ def test_fused_append_every_epilogue(model, tokens):
     braidinfer_amd.check_device_status()
 
 
-@pytest.mark.parametrize("tile", ["2", "3", "1", "128"])
+LLAMA_D32 = dict(hidden=1024, hq=12, hkv=2, d=32, qwen=False)
+QWEN_D32 = dict(hidden=1024, hq=8, hkv=4, d=32, qwen=True)
+
+
+@pytest.mark.parametrize("tile", [2, 3, 1, 128, 64])
 def test_fused_append_tile_forms(tuning, tile):
-    tuning("QKV_TILE", int(tile))
-    c = make_case(50 + int(tile), 300, **LLAMA)
+    """head_dim 32: the tiles of qkv_gemm_kernel, whose workgroups find their rows'
+    slots before the K loop."""
+    tuning("QKV_TILE", tile)
+    c = make_case(50 + tile, 300, **LLAMA_D32)
     check(c, f"tile {tile}")
-    c = make_case(60 + int(tile), 300, **QWEN)
+    c = make_case(60 + tile, 300, **QWEN_D32)
     check(c, f"qwen3 tile {tile}")
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("qwen", [False, True])
+def test_fused_append_register_staged(d, qwen):
+    """K not a multiple of 64: operands through registers, the same epilogue."""
+    c = make_case(70 + d + qwen, 300, hidden=272, hq=4, hkv=2, d=d, qwen=qwen)
+    check(c, f"register-staged D={d}")
 
 
 @pytest.mark.parametrize("tokens", [3, 33, 257])

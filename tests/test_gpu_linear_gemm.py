@@ -87,6 +87,27 @@ def test_general_forms_on_every_tile(tuning, tile, splits):
                  (x.float() @ w.float().t() + r.float()).half().to(x.dtype), what=f"attention output tile={tile}")
 
 
+@pytest.mark.parametrize("n", [2000, 2003])
+def test_whole_and_split_tiles_in_one_call(tuning, n):
+    """18 x 16 tiles of 64 x 128: 256 whole ones, 32 split in three, the last row and
+    column tiles ragged; n = 2003 through the general epilogue."""
+    tuning("GEMM_TILE", 7)
+    tuning("GEMM_SPLITS", 3)
+    g = gen(4400 + n)
+    t, k = 1100, 256
+    assert _lib.workspace_size("bfa_linear_workspace_size", t, k, n, _lib.LINEAR_PLAIN) == 32 * 3 * 64 * 128 * 4
+    x, w, r = randn(g, t, k), randn(g, n, k, std=0.03), randn(g, t, n, std=2.0)
+    slack = 2.0 ** -7 * R.linear(x, w).float().abs()  # one bf16 ulp of the projection, as in test_tiles
+    assert_close(linear_add_residual(x.to(DEV), w.to(DEV), r.to(DEV)), R.linear_add_residual(x, w, r),
+                 what=f"residual n={n}", slack=slack, max_slack_frac=1e-3)
+    inter = n // 2
+    assert _lib.workspace_size("bfa_linear_workspace_size", t, k, inter, 1) == 32 * 3 * 64 * 128 * 4
+    w2 = randn(g, 2 * inter, k, std=0.05)
+    exp = R.gate_up_silu_and_mul(x, w2)
+    assert_close(gate_up_silu_and_mul(x.to(DEV), w2.to(DEV)), exp, what=f"gate_up n={inter}",
+                 slack=2.0 ** -6 * exp.float().abs(), max_slack_frac=1e-4)
+
+
 def test_without_workspace():
     """A caller that brings no workspace gets the unsplit plan: the same result
     up to the order of the fp32 sums, so at most one bf16 rounding apart."""

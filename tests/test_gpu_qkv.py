@@ -318,12 +318,12 @@ def test_prefill_raw_epilogue_256_tiles():
 
 @pytest.mark.parametrize("tile", [2, 3])
 @pytest.mark.parametrize("h", [64, 192, 320, 448])
-@pytest.mark.parametrize("d,hq,hkv", [(128, 4, 2), (80, 6, 2)])
+@pytest.mark.parametrize("d,hq,hkv", [(32, 17, 4), (80, 6, 2)])
 def test_prefill_16x16_stage_counts(tuning, tile, h, d, hq, hkv):
     """The 64-deep DMA loop of the 256x256 (tile 2) and 128x256 8-wave (tile 3)
     tiles, which multiplies 16x16x32 blocks: 1, 3, 5 and 7 stages (the odd tail
     after the two-stage loop), ragged rows and column tiles, through the fused
-    epilogue (head_dim 128, with RoPE) and the raw fp32 store plus the row
+    epilogue (head_dim 32, with RoPE) and the raw fp32 store plus the row
     epilogue (head_dim 80), each against the oracle."""
     tuning("QKV_TILE", tile)
     t = 300
@@ -331,7 +331,7 @@ def test_prefill_16x16_stage_counts(tuning, tile, h, d, hq, hkv):
     q, k, v = FusedRMSNormQKV.forward(x.to(DEV), ln.to(DEV), w.to(DEV), hq, hkv, eps=1e-6)
     for got, exp, name in zip((q, k, v), R.split_qkv(R.qkv_production(x, ln, w, 1e-6), hq, hkv), "qkv"):
         assert_close(got, exp, what=f"16x16 production {name} tile={tile} h={h} d={d}")
-    if d == 128:
+    if d == 32:
         pos = torch.randint(0, 4096, (t,), generator=g)
         cache = R.cos_sin_cache(d, 4096, 1e4)
         q, k, v = llama_attention_input(x.to(DEV), ln.to(DEV), w.to(DEV), hq, hkv, 1e-5, pos.to(DEV),
@@ -372,15 +372,19 @@ def test_prefill_8192_sampled_rows(chain):
                      slack=None if sl is None else sl.reshape(exp.shape))
 
 
-@pytest.mark.parametrize("tile", [None, 128, 64])
-@pytest.mark.parametrize("t,h,hq,hkv,d", [
-    (512, 2048, 32, 4, 64),   # TinyLlama prefill: the planner takes 128x64 (160 tiles)
-    (300, 512, 8, 2, 32),     # head_dim 32 (two heads per 64-column wave), ragged rows
-    (1100, 1024, 8, 4, 64),   # nine row tiles, the last one ragged
+@pytest.mark.parametrize("tile,t,h,hq,hkv,d", [
+    *[(tile, *shape) for tile in (None, 128, 64, 1, 2, 3) for shape in (
+        (300, 512, 8, 2, 32),     # two heads per 64-column wave, ragged rows
+        (512, 2048, 33, 4, 32),   # 41 heads: the last column tile partly empty
+        (1100, 1024, 8, 4, 32),   # nine row tiles, the last one ragged
+    )],
+    (None, 512, 2048, 32, 4, 64),   # TinyLlama prefill
+    (None, 1100, 1024, 8, 4, 64),
 ])
 def test_prefill_narrow_tile(tuning, tile, t, h, hq, hkv, d):
-    """The 128x64 tile (head_dim <= 64 under 128 tiles of 128x128; 8 lanes per
-    row in the fused epilogue) and the 128x128 form it replaces, each against
+    """The 128x64 tile (head_dim 32 under 128 tiles of 128x128, the planner's choice
+    for these; 8 lanes per row in the fused epilogue) and every tile it can be
+    replaced by, and head_dim 64 at the same sizes, each against
     the oracle: the Llama chain, a q/k-norm chain with extreme k_norm weights
     (rope_flip_slack as in test_qwen3_chain) and the mixed variant with bias."""
     tuning("QKV_TILE", tile)

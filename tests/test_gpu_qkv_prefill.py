@@ -8,11 +8,12 @@ import pytest
 import torch
 
 import braidinfer_amd
+from braidinfer_amd import _lib
 from braidinfer_amd.kernels import FusedRMSNormQKVMixedPrecision, PagedKVAppend
 from braidinfer_amd.layers import llama_attention_input, qwen3_attention_input
 from oracle import torch_ref as R
 from tests.helpers import assert_close, bits, randn
-from tests.test_gpu_fused_append import call, make_case, run_case, to_dev
+from tests.test_gpu_fused_append import call, check, make_case, run_case, to_dev
 from tests.test_gpu_qkv import make
 
 pytestmark = pytest.mark.gpu
@@ -44,6 +45,34 @@ def test_tiles(tuning, tile, splits, d, hq, hkv):
         ref = R.qwen3_attention_input(x, ln, w, b, hq, hkv, 1e-6, pos, cache, qn, kn)
         for y, exp, name in zip(got, ref, "qkv"):
             assert_close(y, exp, what=f"qwen3 {name} tile={tile} t={t}", slack=2.0 ** -7 * exp.float().abs() + 2e-2)
+    braidinfer_amd.check_device_status()
+
+
+@pytest.mark.parametrize("d,hq,hkv,split_tiles", [(64, 27, 2, 32), (128, 11, 2, 14)])
+def test_whole_and_split_tiles_in_one_call(tuning, d, hq, hkv, split_tiles):
+    """18 row tiles of 64 tokens, the last one ragged, by 16 (31 heads of 64: half
+    of the last one empty) or 15 column tiles of 128: 256 whole ones, the others
+    split in three; with and without q/k norm, and with the append."""
+    tuning("GEMM_TILE", 7)
+    tuning("GEMM_SPLITS", 3)
+    t, h = 1100, 256
+    n = (hq + 2 * hkv) * d
+    size = _lib.workspace_size("bfa_fused_rmsnorm_qkv_workspace_size", t, h, n, d)
+    assert size == t * h * 2 + split_tiles * 3 * 64 * 128 * 4
+    g, x, ln, w, b = make(570 + d, t, h, hq, hkv, d)
+    pos = torch.randint(-50, 4096, (t,), generator=g)
+    cache = R.cos_sin_cache(d, 4096, 1e4)
+    got = llama_attention_input(x.to(DEV), ln.to(DEV), w.to(DEV), hq, hkv, 1e-5, pos.to(DEV), cache.to(DEV))
+    for y, exp, name in zip(got, R.llama_attention_input(x, ln, w, hq, hkv, 1e-5, pos, cache), "qkv"):
+        assert_close(y, exp, what=f"llama {name} d={d}")
+    qn, kn = randn(g, d, mean=1.0, std=0.1), randn(g, d, mean=1.0, std=0.1)
+    got = qwen3_attention_input(x.to(DEV), ln.to(DEV), w.to(DEV), b.to(DEV), hq, hkv, 1e-6, pos.to(DEV),
+                                cache.to(DEV), qn.to(DEV), kn.to(DEV))
+    ref = R.qwen3_attention_input(x, ln, w, b, hq, hkv, 1e-6, pos, cache, qn, kn)
+    for y, exp, name in zip(got, ref, "qkv"):  # the slack of test_tiles
+        assert_close(y, exp, what=f"qwen3 {name} d={d}", slack=2.0 ** -7 * exp.float().abs() + 2e-2)
+    for qwen in (False, True):
+        check(make_case(580 + d + qwen, t, hidden=h, hq=hq, hkv=hkv, d=d, qwen=qwen), f"append d={d} qwen={qwen}")
     braidinfer_amd.check_device_status()
 
 

@@ -1,8 +1,8 @@
-"""Scratch buffers, between host threads and where memory ends: a buffer is kept per (device, stream) and
-a call queues several kernels over it with the GIL released, so two threads on
-one stream must not interleave theirs; the partial sums of a linear layer above 64
-tokens are optional.  On the CPU, with entry points that only
-record; the GPU counterpart is tests/test_gpu_threads.py."""
+"""Scratch buffers, between host threads and where memory ends.  A buffer is kept
+per (device, stream) and a call queues several kernels over it with the GIL
+released, so two threads on one stream must not interleave theirs; the partial
+sums of a linear layer above 64 tokens are optional.  On the CPU, with entry points
+that only record; the GPU counterpart is tests/test_gpu_threads.py."""
 from __future__ import annotations
 
 import threading
