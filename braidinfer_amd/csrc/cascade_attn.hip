@@ -691,7 +691,9 @@ __global__ __launch_bounds__(256, 2) void cascade_flat_kernel(CasArgs a, FlatArg
   const float sl2 = fabsf(a.scale * 1.4426950408889634f);
   const uint32_t flip = a.scale < 0.f ? 0x80008000u : 0u;
   uint4 qf[RB][QJ];
-  int32_t qp[RB];             // query position, in the key positions' 32 bits
+  // first hidden key position: one past the query's, in the key positions' 32 bits
+  // (INT32_MAX marks an unused slot: always hidden)
+  int32_t qh[RB];
   int32_t qmin = INT32_MAX, qmax = INT32_MIN;  // over the wave's rows
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
@@ -706,11 +708,11 @@ __global__ __launch_bounds__(256, 2) void cascade_flat_kernel(CasArgs a, FlatArg
     int64_t pos = INT32_MAX - 1;  // without a causal mask every key is seen
     if (a.causal)
       pos = a.qpos_i64 ? static_cast<const int64_t*>(a.qpos)[t] : static_cast<const int32_t*>(a.qpos)[t];
-    qp[rb] = static_cast<int32_t>(max(min(pos, static_cast<int64_t>(INT32_MAX - 1)), static_cast<int64_t>(INT32_MIN)));
+    qh[rb] = static_cast<int32_t>(max(min(pos, static_cast<int64_t>(INT32_MAX - 1)), static_cast<int64_t>(INT32_MIN) - 1) + 1);
   }
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
-    int32_t lo = qp[rb], hi = qp[rb];
+    int32_t lo = qh[rb], hi = qh[rb];
 #pragma unroll
     for (int d = 1; d < 16; d *= 2) {
       lo = min(lo, __shfl_xor(lo, d));
@@ -780,7 +782,7 @@ __global__ __launch_bounds__(256, 2) void cascade_flat_kernel(CasArgs a, FlatArg
     };
     // times the scale, then masked: a masked score is -inf whatever the scale
     auto weigh = [&](int32_t kp, cas_f32x4_t (&s)[RB][4]) {
-      const bool edge = __any(kp > qmin);
+      const bool edge = __any(kp >= qmin);
 #pragma unroll
       for (int c = 0; c < 4; ++c)
 #pragma unroll
@@ -792,7 +794,7 @@ __global__ __launch_bounds__(256, 2) void cascade_flat_kernel(CasArgs a, FlatArg
         for (int i = 0; i < 4; ++i) {
           const int32_t kq = __shfl(kp, 16 * c + 4 * (lane >> 4) + i);
 #pragma unroll
-          for (int rb = 0; rb < RB; ++rb) s[rb][c][i] = kq > qp[rb] ? -INFINITY : s[rb][c][i];
+          for (int rb = 0; rb < RB; ++rb) s[rb][c][i] = kq >= qh[rb] ? -INFINITY : s[rb][c][i];
         }
     };
     auto tile_max = [&](const cas_f32x4_t (&s)[4]) {
@@ -831,7 +833,7 @@ __global__ __launch_bounds__(256, 2) void cascade_flat_kernel(CasArgs a, FlatArg
         issue_k(t + 1, b ^ 1);
         issue_v(t + 1, b ^ 1);
       }
-      if (!__all(kp > qmax)) {  // (all: no row of the wave sees a key of the tile)
+      if (!__all(kp >= qmax)) {  // (all: no row of the wave sees a key of the tile)
         scores(kbuf[b], sc);
         weigh(kp, sc);
         uint4 pf[RB][2];

@@ -128,3 +128,22 @@ def test_scores_of_any_size(tuning, tokens, flat, dtype):
         seen = size[: int(qpos[t]) + 1]
         exp[t] = v[: seen.numel()][seen == seen.max()].mean(0)  # equal keys share the weight
     assert_close(out.reshape(tokens, hq, d), exp.repeat_interleave(hq // hkv, 1), what=f"scores of any size {dtype}")
+
+
+def test_positions_at_the_end_of_32_bits(tuning):
+    """Keys from -2^31 on (the flat form keeps key positions in 32 bits): a query
+    below all of them sees none, one at -2^31 + 5 sees six."""
+    tuning("CASCADE_FLAT", 1)
+    hq, hkv, d, ps, tokens = 8, 4, 128, 16, 100
+    chunks, kv, total = build_case(99, hq, hkv, [130, 70], [0, 0], pages=30)
+    att = CascadeAttention(hq, d, 0.0, hkv, ps, rotary_emb=RotaryEmbedding(d, d, 4096, 1e6).to(DEV))
+    levels = att.create_cascade_levels(chunks)
+    q = randn(gen(100), tokens, hq, d).to(DEV)
+    qpos = torch.full((tokens,), -2 ** 31 + 5, device=DEV)
+    qpos[:50] = -2 ** 31 - 7
+    att._plan(levels, att._chunk_meta(levels), q.device)[1].add_(-2 ** 31)  # the plan's key positions, as kept
+    out = att.forward(q, qpos, kv.to(DEV), levels, 0).reshape(tokens, hq, d)
+    CascadeAttention._plans.clear()  # (the changed plan among them)
+    v = kv[chunks[0].page_table[0], 1, :, :6].double().mean(1).repeat_interleave(hq // hkv, 0)
+    assert not out[:50].any()
+    assert_close(out[50:], v.expand(50, -1, -1), what="the first six keys")
