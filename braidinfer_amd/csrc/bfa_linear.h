@@ -28,6 +28,7 @@ struct LinArgs {
   float* part;  // split-K partial tiles
   // (set by the launcher)
   int tiles_m, tiles_n, full, splits, kt;
+  int pairs;  // out takes 4-byte stores at even columns
 };
 
 // The plan for m tokens and n output columns (2 n weight rows with swiglu);

@@ -82,7 +82,7 @@ __device__ __forceinline__ void lin_finish(const LinArgs& q, int64_t row, int64_
 // through the LDS, a few at a time, and walks their rows in a loop.  In registers
 // its code, once per block, outgrew the unroller: the accumulators went to scratch,
 // in the main loop too (3000 tokens, K 2048, n = 8004 951 us, against 147 on the
-// projection GEMM's tiles; 127 like this).  A block is 16 tokens of 16 granules of
+// projection GEMM's tiles; 120 like this).  A block is 16 tokens of 16 granules of
 // 4 values, granule G of token r at G ^ r (a lane writes 4 granules of one token):
 // plain, the wave's 64 columns in order; SwiGLU, its 32 gate columns, then its 32
 // up columns.
@@ -105,10 +105,74 @@ __device__ __forceinline__ float lin_value(const LinArgs& q, float a, float u, f
   }
 }
 
-// `rows` staged tokens of a wave, the first one row0, its first output column c0.
-// Rows that take 16-byte accesses: eight columns a lane; else one, so that the
-// wave's accesses lie next to each other.  A lane keeps its columns, so it reads the
-// bias once; the residual of the next rows is on its way during these rows' work.
+// `rows` staged tokens of a wave, the first one row0, its first output column c0,
+// where output rows take 4-byte accesses of 16-bit elements (W = 2 columns a lane:
+// gate_up of 3000 tokens, K 256, 8004 columns 82 -> 69 us) or none (W = 1): the
+// wave's accesses lie next to each other.  A lane keeps its
+// columns, so it reads the bias once; the residual of the next rows is on its way
+// during these rows' work.
+template <bool SWIGLU, int W>
+__device__ __forceinline__ void lin_rows_narrow(const LinArgs& q, int64_t row0, int64_t c0,
+                                                const gemm_f32x4_t* staged, int rows, int lane) {
+  constexpr int LPR = (SWIGLU ? 32 : 64) / W, STEP = 64 / LPR, U = 8 / W;  // lanes per row; U steps at a time
+  const float* f = reinterpret_cast<const float*>(staged);
+  const int col = lane % LPR * W;
+  const int64_t c = c0 + col;
+  if (c >= q.n) return;
+  const bool whole = c + W <= q.n;
+  float bias[W] = {};
+  if (!SWIGLU && q.bias) {
+#pragma unroll
+    for (int w = 0; w < W; ++w) bias[w] = load_any(q.bias, q.bias_dt, min(c + w, q.n - 1));
+  }
+  struct Res {
+    uint32_t v[U][W];
+  };
+  auto load_res = [&](int t) {
+    Res d{};
+    if (!SWIGLU && q.res) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int w = 0; w < W; ++w)
+          d.v[u][w] = ld_word(q.res, q.res_dt, (row0 + min(t + u * STEP, rows - 1)) * q.ldr + min(c + w, q.n - 1));
+    }
+    return d;
+  };
+  Res cur = load_res(lane / LPR);
+  for (int t0 = lane / LPR; t0 < rows; t0 += U * STEP) {
+    const Res next = load_res(t0 + U * STEP);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int t = t0 + u * STEP;
+      if (t >= rows) break;
+      const int r = t & 15, o = t * 64 + (col & 3);
+      const float* a = f + o + 4 * ((col >> 2) ^ r);
+      const float* up = SWIGLU ? f + o + 4 * ((8 + (col >> 2)) ^ r) : a;
+      float y[W];
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        const int64_t i = (row0 + t) * q.ldr + min(c + w, q.n - 1);
+        const float res = !SWIGLU && q.res ? word_value(cur.v[u][w], q.res_dt, q.res, i) : 0.f;
+        y[w] = lin_value<SWIGLU>(q, a[w], up[w], bias[w], res);
+      }
+      const int64_t i = (row0 + t) * q.ldo + c;
+      if constexpr (W == 2) {
+        if (whole) {
+          const uint32_t b = pack_bf16x2(y[0], y[1]);
+          const uint32_t h = Elem<BFA_DTYPE_F16>::from_f32(y[0]) |
+                             (static_cast<uint32_t>(Elem<BFA_DTYPE_F16>::from_f32(y[1])) << 16);
+          *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(q.out) + i) = q.out_dt == BFA_DTYPE_BF16 ? b : h;
+          continue;
+        }
+      }
+      store_any(q.out, q.out_dt, i, y[0]);
+    }
+    cur = next;
+  }
+}
+
+// Rows that take 16-byte accesses: eight columns a lane; else lin_rows_narrow.
 template <bool SWIGLU>
 __device__ __forceinline__ void lin_rows(const LinArgs& q, int64_t row0, int64_t c0, const gemm_f32x4_t* staged,
                                          int rows, int lane) {
@@ -173,37 +237,8 @@ __device__ __forceinline__ void lin_rows(const LinArgs& q, int64_t row0, int64_t
     }
     return;
   }
-  constexpr int STEP = 64 / COLS, U = 8;  // rows at a time
-  const float* f = reinterpret_cast<const float*>(staged);
-  const int col = lane % COLS;
-  const int64_t c = c0 + col;
-  if (c >= q.n) return;
-  const float bias = !SWIGLU && q.bias ? load_any(q.bias, q.bias_dt, c) : 0.f;
-  struct Res {
-    uint32_t v[U];
-  };
-  auto load_res = [&](int t) {
-    Res d{};
-    if (!SWIGLU && q.res) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) d.v[u] = ld_word(q.res, q.res_dt, (row0 + min(t + u * STEP, rows - 1)) * q.ldr + c);
-    }
-    return d;
-  };
-  Res cur = load_res(lane / COLS);
-  for (int t0 = lane / COLS; t0 < rows; t0 += U * STEP) {
-    const Res next = load_res(t0 + U * STEP);
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int t = t0 + u * STEP;
-      if (t >= rows) break;
-      const int r = t & 15, o = t * 64 + (col & 3);
-      const float a = f[o + 4 * ((col >> 2) ^ r)], up = SWIGLU ? f[o + 4 * ((8 + (col >> 2)) ^ r)] : a;
-      const float res = !SWIGLU && q.res ? word_value(cur.v[u], q.res_dt, q.res, (row0 + t) * q.ldr + c) : 0.f;
-      store_any(q.out, q.out_dt, (row0 + t) * q.ldo + c, lin_value<SWIGLU>(q, a, up, bias, res));
-    }
-    cur = next;
-  }
+  if (q.pairs) lin_rows_narrow<SWIGLU, 2>(q, row0, c0, staged, rows, lane);
+  else lin_rows_narrow<SWIGLU, 1>(q, row0, c0, staged, rows, lane);
 }
 
 // The lane's residual elements, ahead of their use (columns past n are clamped;
@@ -348,6 +383,7 @@ void launch_linear_gemm(const GemmPlan& p, LinArgs q, int dt, hipStream_t st) {
   q.full = p.full;
   q.splits = p.splits;
   q.kt = static_cast<int>(q.k / 64);
+  q.pairs = q.out_dt != BFA_DTYPE_F32 && q.ldo % 2 == 0 && reinterpret_cast<uintptr_t>(q.out) % 4 == 0;
   // (the sum's own rounding is fp32's, none, or the output's)
   const bool same = q.vec && q.n % 8 == 0 && q.proj_dt == dt && q.out_dt == dt &&
                     (q.swiglu || ((q.mid_dt == dt || q.mid_dt == BFA_DTYPE_F32) && (!q.res || q.res_dt == dt)));
