@@ -1616,16 +1616,21 @@ static FlatPlan flat_plan(int64_t rows, int64_t hkv, int64_t num_entries, int64_
   // Two 16-row blocks per wave halve the workgroups, each of which takes 1.1 to 1.7
   // times as long: from more than 256 rows (head_dim 64: 1024), where that saves a
   // round of what the chip holds at once (2 workgroups per CU, head_dim 64: 4) and
-  // there are some tiles to walk, or where the walk is long.  Graph-replayed, one
-  // block and two: Qwen3 600 rows over 8000 keys 75.6 and 60.2 us, 512 over 400
-  // 21.9 and 24.3; Llama-3-8B 4000 over 8000 237 and 206, 300 over 4000 32.9 and
-  // 36.0; TinyLlama 8000 over 8000 138 and 123, 1600 over 8000 41.9 and 52.1.  Of
-  // 402 shapes (100 to 8000 keys, 1 to 8 kv heads) 9 are slower than with one block
-  // at every size, by up to 6 %.
+  // there are some tiles to walk; where the walk is long at head_dim 64; and at
+  // head_dim 128 for 8 row blocks of 64 and fewer, if even, as neighbouring
+  // workgroups are on different XCDs and each of these reads the K and V tiles of
+  // its own.  Graph-replayed, one block and two: Qwen3 600 rows over 8000 keys 75.6
+  // and 60.2 us, 512 over 4000 40.2 and 36.0, 512 over 400 21.9 and 24.3, 1024 over
+  // 4000 48.9 and 51.1; Llama-3-8B 4000 over 8000 237 and 206, 300 over 4000 32.9
+  // and 36.0; TinyLlama 8000 over 8000 138 and 123, 1600 over 8000 41.9 and 52.1.
+  // Of 402 shapes (100 to 8000 keys, 1 to 8 kv heads) 4 are slower than with one
+  // block at every size, by up to 6 %.
   const int64_t held = d == 64 ? 1024 : 512, w1 = blocks * fp.splits, w2 = cdiv(rows, 128) * hkv * fp.splits;
   const int64_t walk = w2 * fp.tiles_per_split;
-  fp.rb = rows > (d == 64 ? 1024 : 256) && ((walk >= 1400 && cdiv(w2, held) < cdiv(w1, held)) ||
-                                            walk >= (d == 64 ? 16000 : 3500)) ? 2 : 1;
+  const bool saves = cdiv(w2, held) < cdiv(w1, held) && walk >= 1400;
+  const bool two = d == 64 ? rows > 1024 && (saves || walk >= 16000)
+                           : rows > 256 && (saves || (rows <= 512 && 2 * w2 == w1 && walk >= 2000));
+  fp.rb = two ? 2 : 1;
   if (tuning(BFA_TUNE_CASCADE_FLAT) == 2) fp.rb = 2;
   fp.part_bytes = fp.splits > 1 ? align256c(fp.splits * hkv * rows * (d + 2) * 4) : 0;
   fp.kf_bytes = align256c(hkv * fp.npad * d * 2);
