@@ -71,23 +71,22 @@ __device__ __forceinline__ float round_sel(float v, int dt) {
 }
 
 // Epilogue dtype forms of the GEMM kernels.  EDT_RT reads every rounding and
-// store dtype from QkvEpi at run time .  The fixed forms compile the dtypes in for
+// store dtype from QkvEpi at run time.  The fixed forms compile the dtypes in for
 // the two combinations the decoders run, so a rounding is one conversion:
 //   EDT_F32_BF16  fp32 projection, no q/k norm, RoPE in fp32, bf16 store
 //                 (the Llama chain: minimal_f32 -> rotary_emb -> .to(bf16))
-//   EDT_BF16      every rounding point bf16 (the Qwen3 chain, the bf16 linears)
+//   EDT_BF16      every rounding point bf16 (the Qwen3 chain)
 //   EDT_F32_F16   the Llama chain with an fp16 store (qkv_prefill.hip)
 enum { EDT_RT = 0, EDT_F32_BF16 = 1, EDT_BF16 = 2, EDT_F32_F16 = 3 };
-template <int EDT> struct QkvDt { static constexpr int Q = -1, N = -1, A = -1, O = -1, M = -1; };
+template <int EDT> struct QkvDt { static constexpr int Q = -1, N = -1, A = -1, O = -1; };
 template <> struct QkvDt<EDT_F32_BF16> {
-  static constexpr int Q = BFA_DTYPE_F32, N = -1, A = BFA_DTYPE_F32, O = BFA_DTYPE_BF16, M = -1;
+  static constexpr int Q = BFA_DTYPE_F32, N = -1, A = BFA_DTYPE_F32, O = BFA_DTYPE_BF16;
 };
 template <> struct QkvDt<EDT_F32_F16> {
-  static constexpr int Q = BFA_DTYPE_F32, N = -1, A = BFA_DTYPE_F32, O = BFA_DTYPE_F16, M = -1;
+  static constexpr int Q = BFA_DTYPE_F32, N = -1, A = BFA_DTYPE_F32, O = BFA_DTYPE_F16;
 };
 template <> struct QkvDt<EDT_BF16> {
-  static constexpr int Q = BFA_DTYPE_BF16, N = BFA_DTYPE_BF16, A = BFA_DTYPE_BF16,
-                       O = BFA_DTYPE_BF16, M = BFA_DTYPE_BF16;
+  static constexpr int Q = BFA_DTYPE_BF16, N = BFA_DTYPE_BF16, A = BFA_DTYPE_BF16, O = BFA_DTYPE_BF16;
 };
 
 __device__ __forceinline__ float round_to(float v, int dt) {

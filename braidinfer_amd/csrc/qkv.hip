@@ -505,7 +505,7 @@ __device__ __forceinline__ void gemm_epilogue(ACC& acc, uint4* lds, const GemmAr
             }
 #pragma unroll
             for (int t = 0; t < 8; ++t)
-              y[t] = rnd<DT::O>(rnd<DT::M>(rnd<DT::Q>(av[t] + bv[t], e.qkv_dt) + rv[t], e.mid_dt), e.out_dt);
+              y[t] = rnd<DT::O>(rnd<-1>(rnd<DT::Q>(av[t] + bv[t], e.qkv_dt) + rv[t], e.mid_dt), e.out_dt);
           }
           if (row < g.m) {
             if (e.vec && col + 8 <= g.n) {
