@@ -63,7 +63,9 @@ const char* bfa_last_error(void);
 #define BFA_TUNE_DECODE_KS 0         /* BFA_DECODE_KS: 64-deep K segments per decode split (1..8) */
 #define BFA_TUNE_DECODE_WG 1         /* BFA_DECODE_WG: workgroup target of the deep-K decode form */
 #define BFA_TUNE_DECODE_SPLITS 2     /* BFA_DECODE_SPLITS: split count of the deep-K decode form */
-#define BFA_TUNE_QKV_TILE 3          /* BFA_QKV_TILE: prefill tile, 1 2 3 64 or 128 (64: head_dim <= 64) */
+#define BFA_TUNE_QKV_TILE 3          /* BFA_QKV_TILE: tile of the QKV prefill GEMM outside
+                                        qkv_prefill.hip (head_dim 32, and raw projections):
+                                        1 2 3 128, or 64 (head_dim 32) */
 #define BFA_TUNE_EDT_RT 4            /* BFA_EDT_RT: non-zero = run-time epilogue dtypes only */
 #define BFA_TUNE_DECODE_PAIR 5       /* BFA_DECODE_PAIR: 0 = never the column-pair decode
                                         kernel, 1 = at any shape it supports */
@@ -74,15 +76,15 @@ const char* bfa_last_error(void);
                                         row blocks per wave */
 #define BFA_TUNE_CASCADE_FLAT_WG 9   /* BFA_CASCADE_FLAT_WG: flat-form workgroup target */
 #define BFA_TUNE_STREAM_STORES 10    /* BFA_STREAM_STORES: 0 = no nontemporal stores */
-#define BFA_TUNE_QKV_PERSIST 11      /* BFA_QKV_PERSIST: prefill GEMM workgroups per CU that loop
-                                        over the tiles (0 = one workgroup per tile; unset: 1 for
-                                        the 256x256 tile, 0 for the others) */
+#define BFA_TUNE_QKV_PERSIST 11      /* BFA_QKV_PERSIST: that GEMM's workgroups per CU that loop
+                                        over 256x256 tiles (0 = one per tile; unset: 1) */
 #define BFA_TUNE_DECODE_GEMV 12      /* BFA_DECODE_GEMV: 0 = never the one-launch decode kernel
                                         (1-8 tokens without q/k norm) */
-#define BFA_TUNE_GEMM_TILE 13      /* BFA_GEMM_TILE: tile id of the GEMMs above 64 tokens (0-7) */
-#define BFA_TUNE_GEMM_SPLITS 14    /* BFA_GEMM_SPLITS: its K splits */
+#define BFA_TUNE_GEMM_TILE 13        /* BFA_GEMM_TILE: tile of the linear layers and of the QKV
+                                        projection (head_dim 64, 128) above 64 tokens, 0 to 7 */
+#define BFA_TUNE_GEMM_SPLITS 14      /* BFA_GEMM_SPLITS: K splits of their tiles past whole rounds */
 #define BFA_TUNE_LINEAR_GEMV 15      /* BFA_LINEAR_GEMV: 0 = never the one-launch linear kernel,
-                                      non-zero = for every call of up to 64 tokens */
+                                        non-zero = for every call of up to 64 tokens */
 #define BFA_TUNE_COUNT 16
 int bfa_set_tuning(int key, int value);
 int bfa_get_tuning(int key);
